@@ -50,8 +50,9 @@ constexpr uint32_t kLeafMax = 4;          // triangles per leaf at most
 // geometry that merges only a few per iteration, such as sizes growing geometrically, would also
 // make a tree too deep for the traversal stack).
 constexpr int kMaxIterations = 4096;
-// Levels of 4-wide nodes the traversal stack holds (three entries pushed per level).
-constexpr int kMaxLevels = 1 + (kTraversalStackDepth + kTraversalSpill) / 3;
+// Levels of 4-wide nodes at most: every level on the way down pushes up to three stack entries.
+constexpr int kMaxLevels = 33;
+static_assert(3 * kMaxLevels <= kTraversalStackDepth + kTraversalSpill, "the traversal stack holds the deepest tree");
 
 // Spreads the low 21 bits of v to every third bit.
 __device__ __forceinline__ uint64_t spread3(uint32_t v) {

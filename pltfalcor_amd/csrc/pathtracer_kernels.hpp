@@ -656,12 +656,13 @@ PLT_DEV bool ms_sample_vertex(uint32_t tri, float b1, float b2, V3 pos, const Su
 }
 // traceMNEEOccluders (:107-150): closest hits along the shadow ray; each must be a specular
 // transmitter that samples a transmission lobe. Ends after at most maxOcc hits.
+template <bool kLean>
 PLT_DEV bool ms_trace_occluders(const PtScene& sc, V3 org, V3 dir, float tmax, int maxOcc, int maxMSBounces, Rng& sg, MsData& d,
                                 int* stk) {
     const V3 wi = -dir;
     for (;;) {
         const Ray r{org.x, org.y, org.z, dir.x, dir.y, dir.z, 0.f, tmax};
-        const Hit h = traverse<false, kTraversalStackDepth>(sc.tsc, r, stk, kPtBlock);
+        const Hit h = traverse<false, kTraversalStackDepth, kLean>(sc.tsc, r, stk, kPtBlock);
         if (h.tri == kNoHit) return true;
         if (d.count >= maxOcc || d.count >= maxMSBounces) return false;
         const V3 posW = walk_point(org, dir, h.t);
@@ -682,7 +683,7 @@ PLT_DEV bool ms_trace_occluders(const PtScene& sc, V3 org, V3 dir, float tmax, i
 // maxIterations ray casts.
 PLT_DEV bool ms_nee_sample(const PtScene& sc, const PtFrame& fr, V3 visOrg, V3 visDir, float visTmax, V3 origin, V3 lightPos,
                            bool distantLight, V3 lightDir, int maxMSBounces, Rng& sg, MsData& d, int* stk) {
-    if (!ms_trace_occluders(sc, visOrg, visDir, visTmax, int(fr.mnee_max_occluders), maxMSBounces, sg, d, stk)) return false;
+    if (!ms_trace_occluders<true>(sc, visOrg, visDir, visTmax, int(fr.mnee_max_occluders), maxMSBounces, sg, d, stk)) return false;
     if (d.count == 0) return true;
     float beta[kMaxMsOccluders];
 #pragma unroll
@@ -721,7 +722,7 @@ PLT_DEV bool ms_nee_sample(const PtScene& sc, const PtFrame& fr, V3 visOrg, V3 v
                 const float dist = wlength(dirTo);
                 dirTo = wdiv(dirTo, dist);
                 const Ray r{p0.x, p0.y, p0.z, dirTo.x, dirTo.y, dirTo.z, fmaxf(1e-4f, .99f * dist), 1.01f * dist};
-                const Hit ch = traverse<false, kTraversalStackDepth>(sc.tsc, r, stk, kPtBlock);
+                const Hit ch = traverse<false, kTraversalStackDepth, true>(sc.tsc, r, stk, kPtBlock);
                 if (ch.tri == kNoHit || sc.tri_mesh[ch.tri] != sc.tri_mesh[h.tri]) {
                     beta[idx] /= 4.f;
                     continue;
@@ -748,7 +749,7 @@ PLT_DEV bool ms_nee_sample(const PtScene& sc, const PtFrame& fr, V3 visOrg, V3 v
     }
     d.woLast = dir;
     const Ray vr{p.x, p.y, p.z, dir.x, dir.y, dir.z, 1e-4f, dist};
-    return traverse<true, kTraversalStackDepth>(sc.tsc, vr, stk, kPtBlock).tri == kNoHit;
+    return traverse<true, kTraversalStackDepth, true>(sc.tsc, vr, stk, kPtBlock).tri == kNoHit;
 }
 // manifoldForwardUnwind (pltpt_solve.rt.slang:80-93): the beam through the walk's vertices, last first.
 template <int N>
@@ -1000,7 +1001,7 @@ solve_kernel(PtScene sc, PtFrame fr) {
                     const int maxMSBounces = int(fr.max_bounces) - p;
                     if (!doMNEE || maxMSBounces <= 0) {
                         const Ray vr{lsOrigin.x, lsOrigin.y, lsOrigin.z, lsDir.x, lsDir.y, lsDir.z, 0.f, lsDist};
-                        ok = traverse<true, kTraversalStackDepth>(sc.tsc, vr, stk, kPtBlock).tri == kNoHit;
+                        ok = traverse<true, kTraversalStackDepth, true>(sc.tsc, vr, stk, kPtBlock).tri == kNoHit;
                         if (ok && misL) {
                             const float bp = mat_pdf(m, s.f, bounce.wi, lsDir, lam[0]);
                             beam.scale(lsPdf / (lsPdf + bp));

@@ -319,7 +319,7 @@ solve_sample_kernel(PtScene sc, PtFrame fr, SolveBuffers sb) {
                             // the walk's random part (manifoldNEESample up to its Newton iterations,
                             // Manifolds.slangh:165-182); the iterations and the light's visibility draw
                             // no random numbers and are left to the walk kernel
-                            ok = ok && ms_trace_occluders(sc, lsOrigin, lsDir, lsDist, int(fr.mnee_max_occluders), maxMSBounces, sg, ms, stk);
+                            ok = ok && ms_trace_occluders<false>(sc, lsOrigin, lsDir, lsDist, int(fr.mnee_max_occluders), maxMSBounces, sg, ms, stk);
                             ok = ok && !(ms.pdf < 1e-6f);
                         }
                         if (ok) {

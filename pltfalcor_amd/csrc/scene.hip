@@ -69,8 +69,8 @@ void replace_owned(DeviceSceneBuffers& d, void* old, void* now) {
 // Uploads the host tree: nodes as float4 x 8 and triangles in leaf order as (v0, id), (v1, 0),
 // (v2, 0), replacing the tree the scene holds.
 int upload_bvh(const HostScene& hs, DeviceSceneBuffers& d) {
-    // a BVH4 of L levels pushes at most 3 (L - 1) entries; the builder's depth bound keeps L <= 32
-    if (3 * (hs.bvh.max_depth - 1) > kTraversalStackDepth + kTraversalSpill)
+    // a BVH4 of L levels pushes at most 3 L entries; the builder's depth bound keeps L <= 32
+    if (3 * hs.bvh.max_depth > kTraversalStackDepth + kTraversalSpill)
         return set_error(PLT_EINVAL, "BVH depth " + std::to_string(hs.bvh.max_depth) + " exceeds the traversal stack (" +
                                          std::to_string(kTraversalStackDepth + kTraversalSpill) + " entries)");
     std::vector<float4> nodes(hs.bvh.nodes.size() * 8);

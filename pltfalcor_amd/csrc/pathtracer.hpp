@@ -156,7 +156,7 @@ struct SurPath {
 enum : int { kUnwindExact = 0, kUnwindQuery = 1, kUnwindApply = 2 };
 // Deferred manifold walks: the light-sampling kernel stores a walk's starting vertices (everything
 // that draws random numbers: the current vertex's and the occluders' delta-lobe samples) with its
-// event and appends the event's index here; the walk kernel, a persistent grid whose lanes each take
+// event and appends the event's index here; the walk kernel, a persistent grid whose quads of lanes each take
 // the next walk as soon as theirs ends, runs the Newton iterations and the light's visibility, writes
 // the converged vertices and the last direction into the event, or turns it into kEvKindVoid.
 struct WalkQueue {

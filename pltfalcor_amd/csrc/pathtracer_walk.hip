@@ -1,9 +1,16 @@
 // The split solve pass's deferred manifold walks: the persistent walk kernel over the frame's walk
 // queue, sized to fill every CU (12 one-wave blocks per CU: three waves per SIMD, each with up to
-// 168 VGPRs), and the clear of the queue's counters. The kernel's time is the latency chain of its
-// longest walks, so it trades occupancy for registers: at four waves per SIMD (128 VGPRs) it
-// spilled, and every Newton iteration paid the spill reloads' round trips (1080p frame, 5.24M triangles: 3.85 ms at
-// four waves, 3.48 ms at three, 3.59 ms at two).
+// 168 VGPRs), and the clear of the queue's counters.
+//
+// The kernel's time is the serial chain of its longest walks (2 % of them run all 60 iterations), not
+// throughput: with a lane per walk the frame's 70,000 to 90,000 walks filled less than half of the
+// resident lanes, and each of a long walk's casts paid for four box tests and a leaf's triangles one
+// after the other. So a walk has a quad of lanes: a node's four boxes and a leaf's up to four triangles
+// are tested at once (traverse_quad), 16 walks per wave instead of 64 also end a wave's trip sooner, and
+// the Newton steps between casts run in all four lanes alike. Walk kernel, lane -> quad per walk: 1080p
+// frame over 5.24 M triangles 3.25 -> 1.89 ms, 853 x 481 with every light type 3.23 -> 1.46 ms, 96 x 64
+// preview 0.55 -> 0.38 ms; walk vertices bit for bit the same. Registers still count for more than
+// occupancy: at four waves per SIMD (128 VGPRs) every Newton iteration paid for spill reloads.
 #include "pathtracer_split.hpp"
 
 namespace plt {
@@ -21,23 +28,26 @@ PLT_DEV V3 hit_pos(const SolveBuffers& sb, const uint32_t* h) {
               __uint_as_float(h[(kHitPos + 2) * sb.hit_cap]));
 }
 
-// A persistent grid: each lane runs one walk at a time as a sequence of ray casts, and every trip
-// through the loop casts at most one ray per lane. A lane whose walk ends takes the next one from
-// the queue at the top of the next trip, so a wave's lanes stay busy while its longest walk
-// iterates (running whole walks per lane would hold every lane of a wave until its longest walk,
+// A persistent grid: each quad runs one walk at a time as a sequence of ray casts, and every trip
+// through the loop casts at most one ray per quad. A quad whose walk ends takes the next one from
+// the queue at the top of the next trip, so a wave's quads stay busy while its longest walk
+// iterates (running whole walks would hold the wave until its longest walk,
 // up to MNEEMaxIterations casts, had ended). A walk is deterministic given its starting vertices,
-// so which lane runs it, and when, changes nothing in its result.
+// so which quad runs it, and when, changes nothing in its result. The four lanes of a quad hold the
+// same state throughout; each writes the vertices that it reads back itself (same values, same
+// addresses), the first one alone writes the rest.
 //
-// Every lane ends: a lane retires once the queue is empty, and a walk ends after at most
+// Every quad ends: a quad retires once the queue is empty, and a walk ends after at most
 // MNEEMaxIterations line-search casts, one visibility cast and, between casts, at most two passes
 // over its vertices (a pass that casts nothing either meets the threshold at every vertex, which
 // ends the walk, or follows a pass that cast).
 __global__ void __launch_bounds__(kWalkBlock) __attribute__((amdgpu_waves_per_eu(3, 3)))
 solve_walk_kernel(PtScene sc, PtFrame fr, SolveBuffers sb) {
-    __shared__ int stack[kTraversalStackDepth * kWalkBlock];
+    __shared__ int stack[kQuadStack * kQuads];
     __shared__ float betaS[kMaxMsOccluders * kWalkBlock];  // per-vertex step sizes, [vertex][lane]
     const uint32_t lane = threadIdx.x;
-    int* stk = stack + lane;
+    const bool first = (lane & 3u) == 0u;  // the quad's lane that counts and writes what the walk does not read again
+    int* stk = stack + (lane >> 2);
     float* beta = betaS + lane;
     const uint32_t total = sb.walk.counters[0];
     const size_t regionEvents = size_t(kPtBlock) * sb.ev_per_path, regionHits = size_t(kPtBlock) * sb.hits_per_path;
@@ -56,13 +66,17 @@ solve_walk_kernel(PtScene sc, PtFrame fr, SolveBuffers sb) {
     Ray ray{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     uint32_t casts = 0;
     auto finish = [&](bool ok) {
-        if (ok) ev_put3(sb, e, kEvWo, v3(ray.dx, ray.dy, ray.dz));
-        else ev_put(sb, e, kEvMeta, (meta & ~(3u << 13)) | (kEvKindVoid << 13));
+        if (first) {
+            if (ok) ev_put3(sb, e, kEvWo, v3(ray.dx, ray.dy, ray.dz));
+            else ev_put(sb, e, kEvMeta, (meta & ~(3u << 13)) | (kEvKindVoid << 13));
+        }
         state = kWalkIdle;
     };
     for (;;) {
         if (state == kWalkIdle && !retired) {
-            const uint32_t k = wave_append(sb.walk.counters + 1, 1u);
+            uint32_t k = 0;
+            if (first) k = wave_append(sb.walk.counters + 1, 1u);
+            k = quad_first(k);
             if (k >= total) {
                 retired = true;
             } else {
@@ -83,7 +97,7 @@ solve_walk_kernel(PtScene sc, PtFrame fr, SolveBuffers sb) {
                 state = kWalkNewton;
             }
         }
-        if (__ballot(state != kWalkIdle) == 0) break;  // every lane has retired (the whole wave leaves together)
+        if (__ballot(state != kWalkIdle) == 0) break;  // every quad has retired (the whole wave leaves together)
         // advance each walk to its next ray
         bool cast = false;
         if (state == kWalkNewton) {
@@ -160,8 +174,8 @@ solve_walk_kernel(PtScene sc, PtFrame fr, SolveBuffers sb) {
             }
         }
         if (cast) {
-            ++casts;
-            const Hit ch = traverse_rays<kTraversalStackDepth>(sc.tsc, ray, stk, kWalkBlock, state == kWalkVis);
+            casts += first ? 1u : 0u;
+            const Hit ch = traverse_quad(sc.tsc, ray, stk, state == kWalkVis);
             if (state == kWalkVis) {
                 finish(ch.tri == kNoHit);
             } else if (ch.tri == kNoHit || sc.tri_mesh[ch.tri] != hmesh) {

@@ -369,4 +369,82 @@ __device__ __forceinline__ Hit traverse(const TraceScene& sc, const Ray& r, int*
     return kLean ? traverse_rays_lean<kDepth>(sc, r, stack, stride, kAnyHit) : traverse_rays<kDepth>(sc, r, stack, stride, kAnyHit);
 }
 
+// ---------------------------------------------------------------------------------------
+// One ray per quad of lanes: lane i of the quad tests child i of a node and triangle i of a leaf.
+// ---------------------------------------------------------------------------------------
+__device__ __forceinline__ uint32_t quad_xor1(uint32_t v) { return uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0xB1, 0xF, 0xF, true)); }
+__device__ __forceinline__ uint32_t quad_xor2(uint32_t v) { return uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0x4E, 0xF, 0xF, true)); }
+__device__ __forceinline__ uint32_t quad_xor3(uint32_t v) { return uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0x1B, 0xF, 0xF, true)); }
+__device__ __forceinline__ uint32_t quad_first(uint32_t v) { return uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0x00, 0xF, 0xF, true)); }
+// Stack entries of a quad's traversal, all in LDS: three for each of the 33 levels of the deepest tree
+// the builders make, interleaved over the wave's 16 quads ([entry][quad]).
+constexpr int kQuadStack = 100;
+constexpr int kQuads = 16;
+
+// The hit traverse_rays finds for the same ray, cast by the four lanes of a quad together (the ray is
+// the same in all four, and so is the control flow; the result is too). `stack` points at the quad's
+// first slot; its lanes read what the others wrote, in one wave's program order, so the accesses are
+// wavefront-scope atomics (plain LDS instructions that the compiler neither merges nor moves).
+__device__ __forceinline__ Hit traverse_quad(const TraceScene& sc, const Ray& r, int* stack, bool anyHit) {
+    const RayConst c = ray_const(r);
+    const uint32_t sub = __lane_id() & 3u, shift = __lane_id() & 60u;
+    const uint32_t onx = (c.sx >> 2) + sub, ofx = 4u - (c.sx >> 2) + sub;
+    const uint32_t ony = 8u + (c.sy >> 2) + sub, ofy = 12u - (c.sy >> 2) + sub;
+    const uint32_t onz = 16u + (c.sz >> 2) + sub, ofz = 20u - (c.sz >> 2) + sub;
+    const float* nodes = reinterpret_cast<const float*>(sc.nodes);
+    Hit h{kNoHit, 0.f, 0.f, r.tmax};
+    int node = 0, sp = 0;
+    for (;;) {
+        bool next = false;
+        if (node >= 0) {
+            const float* q = nodes + 32 * size_t(uint32_t(node));
+            const float nx = q[onx], fx = q[ofx], ny = q[ony], fy = q[ofy], nz = q[onz], fz = q[ofz];
+            const uint32_t child = __float_as_uint(q[24u + sub]);
+            const uint32_t key = box_key(box_entry(c, nx, fx, ny, fy, nz, fz, h.t), sub);
+            const bool in = key != 0xFFFFFFFFu;
+            // how many children are nearer: 0 goes next, the others on the stack, farthest first
+            const uint32_t rank = (quad_xor1(key) < key ? 1u : 0u) + (quad_xor2(key) < key ? 1u : 0u) + (quad_xor3(key) < key ? 1u : 0u);
+            const int hits = __popc(uint32_t(__ballot(in) >> shift) & 15u);
+            if (in && rank != 0u)
+                __hip_atomic_store(stack + (sp + hits - 1 - int(rank)) * kQuads, int(child), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+            uint32_t sel = in && rank == 0u ? child : 0u;
+            sel |= quad_xor1(sel);
+            sel |= quad_xor2(sel);
+            if (hits > 0) {
+                node = int(sel);
+                sp += hits - 1;
+                next = true;
+            }
+        } else {
+            const uint32_t leaf = uint32_t(~node), cnt = (leaf & 7u) + 1u;
+            const float4* t = sc.tris + 3 * size_t((leaf >> 3) + min(sub, cnt - 1u));
+            const float4 v0 = t[0], v1 = t[1], v2 = t[2];
+            Hit x{kNoHit, 0.f, 0.f, h.t};
+            float tt, b1, b2;
+            const bool ok = intersect_tri(c.p, v0, v1, v2, c.tmin, h.t, tt, b1, b2);
+            if (ok && sub < cnt) x = Hit{__float_as_uint(v0.w), b1, b2, tt};
+            if ((uint32_t(__ballot(x.tri != kNoHit) >> shift) & 15u) != 0u) {
+                // the quad's smallest (t, id), against the closest hit so far
+                auto better = [](Hit& a, const Hit& b) {
+                    if (b.t < a.t || (b.t == a.t && b.tri < a.tri)) a = b;
+                };
+                auto other = [](const Hit& a, auto f) {
+                    return Hit{f(a.tri), __uint_as_float(f(__float_as_uint(a.b1))), __uint_as_float(f(__float_as_uint(a.b2))),
+                               __uint_as_float(f(__float_as_uint(a.t)))};
+                };
+                better(x, other(x, quad_xor1));
+                better(x, other(x, quad_xor2));
+                better(h, x);
+                if (anyHit) return h;
+            }
+        }
+        if (!next) {
+            if (sp == 0) break;
+            --sp;
+            node = __hip_atomic_load(stack + sp * kQuads, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        }
+    }
+    return h;
+}
+
 }  // namespace plt

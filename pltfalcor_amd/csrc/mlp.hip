@@ -1,13 +1,10 @@
 // Learned BSDF surrogate (no counterpart in the reference): a 22-128-128-128-16 ReLU MLP whose
 // forward pass, backward pass and Adam update run on CDNA4 matrix cores.
 //
-// Every product is one NT GEMM, C[M x N] = A[M x K] * Bt[N x K]^T, with both operands bf16 and
-// K-contiguous so that each MFMA fragment (8 consecutive k of one row) is one 16 B load; the
-// activations are kept in both sample-major [batch x features] (forward/backward-data operand) and
-// feature-major [features x batch] (weight-gradient operand) layouts, written by the producing
-// GEMM's epilogue. Accumulation is FP32 (v_mfma_f32_16x16x32_bf16); master weights and Adam
-// moments are FP32; weight gradients are split-K partial sums reduced in a fixed order (the
-// result does not depend on scheduling).
+// Every MFMA operand is bf16 and contiguous along the contracted dimension, so that a fragment (8
+// consecutive k of one row) is one 16 B load. Accumulation is FP32 (v_mfma_f32_16x16x32_bf16); master
+// weights and Adam moments are FP32; weight gradients are partial sums per workgroup reduced in a
+// fixed order (the result does not depend on scheduling).
 //
 // Layers (parameter order of plt_surrogate_params): W1 [128 x 22], b1 [128], W2 [128 x 128], b2,
 // W3 [128 x 128], b3, W4 [16 x 128], b4 [16] = 38,032 FP32 values. Inputs are padded to 32
@@ -16,6 +13,7 @@
 #include <cmath>
 #include <cstring>
 #include <random>
+#include <type_traits>
 #include <vector>
 #include "plt_internal.hpp"
 #include "surrogate.hpp"
@@ -31,35 +29,14 @@ constexpr int kParams = kHid * kIn + kHid + 2 * (kHid * kHid + kHid) + kOut * kH
 static_assert(kParams == 38032, "parameter count");
 
 // ---------------------------------------------------------------------------------------
-// NT GEMM with fused epilogues.
+// Plain NT GEMM, C[M x N] = A[M x K] * Bt[N x K]^T (plt_mlp_gemm_nt).
 // ---------------------------------------------------------------------------------------
-enum Epilogue : int {
-    kEpiF32 = 0,       // Cf[i, j] = acc (+ bias[j])
-    kEpiBiasRelu = 1,  // h = max(acc + bias[j], 0): Cb[i, j] = bf16(h), Ct[j, i] = bf16(h) if Ct
-    kEpiMask = 2,      // g = acc if H[i, j] > 0 else 0: Cb[i, j] = bf16(g), Ct[j, i] = bf16(g) if Ct
-    kEpiPartial = 3,   // Cf[z][i, j] = acc over this split's K range (z = blockIdx.z)
-};
 struct GemmArgs {
-    const __bf16* A;   // [M x K], row stride lda
-    const __bf16* Bt;  // [N x K], row stride ldb
-    int M, N, K, lda, ldb;
-    int epi;
-    const float* bias;
-    float* Cf;
-    __bf16* Cb;
-    __bf16* Ct;
-    const __bf16* H;
-    int ldc, ldt, ldh;
-    int k_per_split;  // K range of one split (multiple of 32)
-    size_t split_stride;
-    // kEpiMask: per-tile column sums of the bf16 outputs (the bias gradient's partials) into
-    // bias_part[blockIdx.y * kBiasCols + bias_col + j] when set
-    float* bias_part;
-    int bias_col;
+    const __bf16* A;   // [M x K]
+    const __bf16* Bt;  // [N x K]
+    int M, N, K;
+    float* C;
 };
-// Columns of the bias-gradient partials: b4 (16, from the loss kernel's 256-sample blocks), then
-// b3, b2, b1 (128 each, from the backward GEMMs' 64-row tiles).
-constexpr int kBiasCols = 16 + 3 * 128;
 
 constexpr int kTile = 64, kKStep = 32, kLdsRow = kKStep + 8;  // +8 bf16 per row breaks bank conflicts
 constexpr int kGemmThreads = 256;
@@ -67,11 +44,8 @@ constexpr int kGemmThreads = 256;
 __global__ void __launch_bounds__(kGemmThreads) gemm_nt_kernel(GemmArgs g) {
     __shared__ __bf16 As[kTile * kLdsRow];
     __shared__ __bf16 Bs[kTile * kLdsRow];
-    __shared__ float colsum[2][kTile];
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
     const int m0 = blockIdx.y * kTile, n0 = blockIdx.x * kTile;
-    const int kbeg = blockIdx.z * g.k_per_split;
-    const int kend = min(g.K, kbeg + g.k_per_split);
     // staging: thread t copies 8 bf16 of row t/4, k offset 8*(t%4), of both tiles
     const int sr = t >> 2, sk = (t & 3) * 8;
     // wave w computes rows 32*(w/2)..+31 and columns 32*(w%2)..+31 of the tile: 2 x 2 MFMA blocks
@@ -82,10 +56,10 @@ __global__ void __launch_bounds__(kGemmThreads) gemm_nt_kernel(GemmArgs g) {
     for (int a = 0; a < 2; ++a)
 #pragma unroll
         for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = kbeg; k0 < kend; k0 += kKStep) {
+    for (int k0 = 0; k0 < g.K; k0 += kKStep) {
         bf16x8 va = {}, vb = {};
-        if (m0 + sr < g.M) va = *reinterpret_cast<const bf16x8*>(g.A + size_t(m0 + sr) * g.lda + k0 + sk);
-        if (n0 + sr < g.N) vb = *reinterpret_cast<const bf16x8*>(g.Bt + size_t(n0 + sr) * g.ldb + k0 + sk);
+        if (m0 + sr < g.M) va = *reinterpret_cast<const bf16x8*>(g.A + size_t(m0 + sr) * g.K + k0 + sk);
+        if (n0 + sr < g.N) vb = *reinterpret_cast<const bf16x8*>(g.Bt + size_t(n0 + sr) * g.K + k0 + sk);
         *reinterpret_cast<bf16x8*>(As + sr * kLdsRow + sk) = va;
         *reinterpret_cast<bf16x8*>(Bs + sr * kLdsRow + sk) = vb;
         __syncthreads();
@@ -101,7 +75,6 @@ __global__ void __launch_bounds__(kGemmThreads) gemm_nt_kernel(GemmArgs g) {
         __syncthreads();
     }
     // D layout of a 16 x 16 block: lane holds rows 4*(lane/16) + r (r = 0..3) of column lane%16
-    float cs[2] = {0.f, 0.f};  // this lane's share of its two columns' sums (kEpiMask)
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -110,53 +83,14 @@ __global__ void __launch_bounds__(kGemmThreads) gemm_nt_kernel(GemmArgs g) {
             for (int r = 0; r < 4; ++r) {
                 const int i = m0 + wr + 16 * a + 4 * (lane >> 4) + r;
                 const int j = n0 + wc + 16 * b + (lane & 15);
-                if (i >= g.M || j >= g.N) continue;
-                float v = acc[a][b][r];
-                switch (g.epi) {
-                    case kEpiF32:
-                        g.Cf[size_t(i) * g.ldc + j] = g.bias ? v + g.bias[j] : v;
-                        break;
-                    case kEpiBiasRelu: {
-                        v = fmaxf(v + g.bias[j], 0.f);
-                        const __bf16 h = static_cast<__bf16>(v);
-                        g.Cb[size_t(i) * g.ldc + j] = h;
-                        if (g.Ct) g.Ct[size_t(j) * g.ldt + i] = h;
-                        break;
-                    }
-                    case kEpiMask: {
-                        const float h = static_cast<float>(g.H[size_t(i) * g.ldh + j]);
-                        const __bf16 d = static_cast<__bf16>(h > 0.f ? v : 0.f);
-                        if (g.Cb) g.Cb[size_t(i) * g.ldc + j] = d;
-                        if (g.Ct) g.Ct[size_t(j) * g.ldt + i] = d;
-                        cs[b] += static_cast<float>(d);
-                        break;
-                    }
-                    default:
-                        g.Cf[blockIdx.z * g.split_stride + size_t(i) * g.ldc + j] = v;
-                        break;
-                }
+                if (i < g.M && j < g.N) g.C[size_t(i) * g.N + j] = acc[a][b][r];
             }
-    if (g.epi == kEpiMask && g.bias_part) {  // block-uniform
-        // the tile's column sums in a fixed order: lanes of one column (xor 16, 32), then the two
-        // waves that share the column range
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            cs[b] += __shfl_xor(cs[b], 16);
-            cs[b] += __shfl_xor(cs[b], 32);
-        }
-        if (lane < 16) {
-            colsum[wave >> 1][wc + lane] = cs[0];
-            colsum[wave >> 1][wc + 16 + lane] = cs[1];
-        }
-        __syncthreads();
-        if (t < kTile && n0 + t < g.N) g.bias_part[size_t(blockIdx.y) * kBiasCols + g.bias_col + n0 + t] = colsum[0][t] + colsum[1][t];
-    }
 }
 
-int gemm(const GemmArgs& g, int splits, hipStream_t st) {
-    if (g.M <= 0 || g.N <= 0 || g.K <= 0 || g.K % kKStep || g.lda % 8 || g.ldb % 8 || g.k_per_split % kKStep)
+int gemm(const GemmArgs& g, hipStream_t st) {
+    if (g.M <= 0 || g.N <= 0 || g.K <= 0 || g.K % kKStep)
         return set_error(PLT_EINVAL, "mlp gemm: shapes must be multiples of 32 (K) and 8 (leading dimensions)");
-    const dim3 grid((g.N + kTile - 1) / kTile, (g.M + kTile - 1) / kTile, splits);
+    const dim3 grid((g.N + kTile - 1) / kTile, (g.M + kTile - 1) / kTile);
     hipLaunchKernelGGL(gemm_nt_kernel, grid, dim3(kGemmThreads), 0, st, g);
     return check_launch("gemm_nt_kernel");
 }
@@ -353,72 +287,6 @@ __global__ void __launch_bounds__(kFThreads) mlp_infer_kernel(int n, const float
 // ---------------------------------------------------------------------------------------
 constexpr int kEw = 256;
 
-// X f32 [n x 22] -> Xb bf16 [n x 32] (zero padded) and, if Xt, Xt [32 x ldt].
-__global__ void pack_inputs_kernel(int n, const float* __restrict__ X, __bf16* __restrict__ Xb, __bf16* __restrict__ Xt, int ldt) {
-    const int i = blockIdx.x * kEw + threadIdx.x;
-    if (i >= n) return;
-    for (int f = 0; f < kInPad; ++f) {
-        const __bf16 v = static_cast<__bf16>(f < kIn ? X[size_t(i) * kIn + f] : 0.f);
-        Xb[size_t(i) * kInPad + f] = v;
-        if (Xt) Xt[size_t(f) * ldt + i] = v;
-    }
-}
-
-// Mean-squared error over the 16 outputs: dL/dY = 2 (Y - T) / (n * 16), stored as bf16 in dY
-// [n x 32] (zero padded) and dYt [16 x ldt]; per-block partial sums of the loss in FP32.
-// The block's column sums of dY (the last layer's bias gradient) go to bias_part[blockIdx.x *
-// kBiasCols + f] in a fixed order (lanes of a wave by xor steps, then the four waves).
-__global__ void loss_grad_kernel(int n, const float* __restrict__ Y, const float* __restrict__ T, __bf16* __restrict__ dY,
-                                 __bf16* __restrict__ dYt, int ldt, float* __restrict__ loss_part, float* __restrict__ bias_part) {
-    __shared__ float red[kEw];
-    __shared__ float colsum[kEw / 64][kOut];
-    const int i = blockIdx.x * kEw + threadIdx.x;
-    float l = 0.f;
-    float gs[kOut];
-#pragma unroll
-    for (int f = 0; f < kOut; ++f) gs[f] = 0.f;
-    if (i < n) {
-        const float s = 2.f / (float(n) * float(kOut));
-#pragma unroll
-        for (int f = 0; f < kOutPad; ++f) {
-            float g = 0.f;
-            if (f < kOut) {
-                const float d = Y[size_t(i) * kOut + f] - T[size_t(i) * kOut + f];
-                l += d * d;
-                g = s * d;
-            }
-            const __bf16 gb = static_cast<__bf16>(g);
-            dY[size_t(i) * kOutPad + f] = gb;
-            if (f < kOut) {
-                dYt[size_t(f) * ldt + i] = gb;
-                gs[f] = static_cast<float>(gb);
-            }
-        }
-    }
-    red[threadIdx.x] = l;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-    for (int f = 0; f < kOut; ++f) {
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) gs[f] += __shfl_xor(gs[f], o);
-    }
-    if (lane == 0) {
-#pragma unroll
-        for (int f = 0; f < kOut; ++f) colsum[wave][f] = gs[f];
-    }
-    __syncthreads();
-    for (int s = kEw / 2; s > 0; s >>= 1) {
-        if (int(threadIdx.x) < s) red[threadIdx.x] += red[threadIdx.x + s];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) loss_part[blockIdx.x] = red[0];
-    if (bias_part && threadIdx.x < kOut) {
-        float c = 0.f;
-        for (int w = 0; w < kEw / 64; ++w) c += colsum[w][threadIdx.x];
-        bias_part[size_t(blockIdx.x) * kBiasCols + threadIdx.x] = c;
-    }
-}
-
 // bf16 operand copies of one layer: W [out x in_pad] and Wt [in x out_pad] from the master
 // weights [out x in] (padding zero).
 __global__ void cast_weights_kernel(int out, int in, int in_pad, int out_pad, const float* __restrict__ Wm, __bf16* __restrict__ W,
@@ -445,7 +313,6 @@ namespace {
 constexpr size_t kOffW1 = 0, kOffB1 = kOffW1 + size_t(kHid) * kIn, kOffW2 = kOffB1 + kHid, kOffB2 = kOffW2 + size_t(kHid) * kHid,
                  kOffW3 = kOffB2 + kHid, kOffB3 = kOffW3 + size_t(kHid) * kHid, kOffW4 = kOffB3 + kHid,
                  kOffB4 = kOffW4 + size_t(kOut) * kHid;
-constexpr int kSplitTarget = 64;  // weight-gradient GEMM splits of the batch (K) dimension
 constexpr size_t kTrainStateWords = 16;
 
 template <class T>
@@ -469,149 +336,6 @@ int cast_all(plt_surrogate* s, hipStream_t st) {
                            s->params + l.off, l.W, l.Wt);
     }
     return check_launch("cast_weights_kernel");
-}
-
-GemmArgs nt(const __bf16* A, int lda, const __bf16* Bt, int ldb, int M, int N, int K) {
-    GemmArgs g{};
-    g.A = A; g.lda = lda; g.Bt = Bt; g.ldb = ldb; g.M = M; g.N = N; g.K = K;
-    g.k_per_split = K;
-    return g;
-}
-
-// Forward pass of n <= max_batch samples already packed in Xb; keeps H1..H3 (and their
-// feature-major copies when `keep_t`) and writes the raw outputs to Y [n x 16] (FP32).
-int forward(plt_surrogate* s, int n, bool keep_t, hipStream_t st) {
-    const int ld = int(s->max_batch);
-    int rc;
-    GemmArgs g = nt(s->Xb, kInPad, s->W1, kInPad, n, kHid, kInPad);
-    g.epi = kEpiBiasRelu; g.bias = s->params + kOffB1; g.Cb = s->H1; g.ldc = kHid; g.Ct = keep_t ? s->H1t : nullptr; g.ldt = ld;
-    if ((rc = gemm(g, 1, st)) < 0) return rc;
-    g = nt(s->H1, kHid, s->W2, kHid, n, kHid, kHid);
-    g.epi = kEpiBiasRelu; g.bias = s->params + kOffB2; g.Cb = s->H2; g.ldc = kHid; g.Ct = keep_t ? s->H2t : nullptr; g.ldt = ld;
-    if ((rc = gemm(g, 1, st)) < 0) return rc;
-    g = nt(s->H2, kHid, s->W3, kHid, n, kHid, kHid);
-    g.epi = kEpiBiasRelu; g.bias = s->params + kOffB3; g.Cb = s->H3; g.ldc = kHid; g.Ct = keep_t ? s->H3t : nullptr; g.ldt = ld;
-    if ((rc = gemm(g, 1, st)) < 0) return rc;
-    g = nt(s->H3, kHid, s->W4, kHid, n, kOut, kHid);
-    g.epi = kEpiF32; g.bias = s->params + kOffB4; g.Cf = s->Y; g.ldc = kOut;
-    return gemm(g, 1, st);
-}
-
-// The weight gradients' split-K partials: region r of s->part holds splits x (out x in) floats of
-// layer 4, 3, 2, 1 in that order (layer 1 with its 32 padded inputs).
-constexpr int kGradCount[4] = {kOut * kHid, kHid * kHid, kHid * kHid, kHid * kInPad};
-constexpr int kGradTotal = kOut * kHid + 2 * kHid * kHid + kHid * kInPad;  // 38,912
-int split_len(int n) { return (n / kKStep + kSplitTarget - 1) / kSplitTarget * kKStep; }
-
-// dW[out x in] = sum over the batch of Gt[out, b] * Ht[in, b] (n a multiple of 32), as split-K
-// partials into the layer's region of s->part; grad_reduce_kernel sums them.
-int weight_grad(plt_surrogate* s, int n, const __bf16* Gt, int out, const __bf16* Ht, int in, size_t region, hipStream_t st) {
-    const int ld = int(s->max_batch);
-    const int per = split_len(n);
-    const int splits = (n + per - 1) / per;
-    GemmArgs g = nt(Gt, ld, Ht, ld, out, in, n);
-    g.epi = kEpiPartial; g.Cf = s->part + region * kSplitTarget; g.ldc = in; g.k_per_split = per; g.split_stride = size_t(out) * in;
-    return gemm(g, splits, st);
-}
-
-// Every gradient from its partials, in one launch. A block takes 64 elements of the
-// [weights..., biases] list with four threads each: thread group g sums the element's partials
-// z = g, g + 4, ... (all loads issued before the adds), and the four sums are combined in order.
-// Weight elements sum their `splits` split-K partials; the kBiasCols bias elements sum their
-// `rows_out` (b4) or `rows_hid` (b3, b2, b1) tile partials. Layer 1 drops its padding.
-constexpr int kReduceLanes = 64, kReduceMax = 16;  // elements per block; partials per thread at most
-__global__ void __launch_bounds__(256) grad_reduce_kernel(int splits, int rows_out, int rows_hid, const float* __restrict__ part,
-                                                          const float* __restrict__ bias_part, float* __restrict__ grads) {
-    __shared__ float sums[4][kReduceLanes];
-    const int el = threadIdx.x & (kReduceLanes - 1), g = threadIdx.x >> 6;
-    const int e = blockIdx.x * kReduceLanes + el;
-    const bool live = e < kGradTotal + kBiasCols;
-    const bool bias = e >= kGradTotal;
-    int count = splits, cnt = 0, local = 0, c = 0;
-    size_t base = 0;
-    if (live && bias) {
-        c = e - kGradTotal;
-        count = c < kOut ? rows_out : rows_hid;
-    } else if (live) {
-        constexpr int c4 = kOut * kHid, c3 = kHid * kHid, c2 = kHid * kHid;
-        const int r = e < c4 ? 0 : e < c4 + c3 ? 1 : e < c4 + c3 + c2 ? 2 : 3;
-        const int first = r == 0 ? 0 : r == 1 ? c4 : r == 2 ? c4 + c3 : c4 + c3 + c2;
-        cnt = r == 0 ? c4 : r == 1 ? c3 : r == 2 ? c2 : kHid * kInPad;
-        local = e - first;
-        base = size_t(first) * kSplitTarget;
-    }
-    float acc = 0.f;
-    if (live) {
-        // up to kReduceMax partials per thread in one batch of loads (weight partials: splits <= 64)
-        for (int z0 = g; z0 < count; z0 += 4 * kReduceMax) {
-            float v[kReduceMax];
-#pragma unroll
-            for (int q = 0; q < kReduceMax; ++q) {
-                const int z = z0 + 4 * q;
-                v[q] = z < count ? (bias ? bias_part[size_t(z) * kBiasCols + c] : part[base + size_t(z) * cnt + local]) : 0.f;
-            }
-#pragma unroll
-            for (int q = 0; q < kReduceMax; ++q) acc += v[q];
-        }
-    }
-    sums[g][el] = acc;
-    __syncthreads();
-    if (g != 0 || !live) return;
-    const float sum = (sums[0][el] + sums[1][el]) + (sums[2][el] + sums[3][el]);
-    if (bias) {
-        const size_t dst = c < kOut ? kOffB4 + c : c < kOut + kHid ? kOffB3 + (c - kOut) : c < kOut + 2 * kHid ? kOffB2 + (c - kOut - kHid)
-                                                                                           : kOffB1 + (c - kOut - 2 * kHid);
-        grads[dst] = sum;
-    } else if (cnt == kHid * kInPad) {
-        if (local % kInPad < kIn) grads[kOffW1 + (local / kInPad) * kIn + local % kInPad] = sum;
-    } else {
-        grads[(cnt == kOut * kHid ? kOffW4 : e < kOut * kHid + kHid * kHid ? kOffW3 : kOffW2) + local] = sum;
-    }
-}
-
-// Loss and gradients of n samples (X packed, T [n x 16] FP32 targets) into s->grads.
-int loss_and_grads(plt_surrogate* s, int n, const float* T, float* loss_host, hipStream_t st) {
-    const int ld = int(s->max_batch);
-    int rc;
-    if ((rc = forward(s, n, true, st)) < 0) return rc;
-    const int blocks = (n + kEw - 1) / kEw;
-    hipLaunchKernelGGL(loss_grad_kernel, dim3(blocks), dim3(kEw), 0, st, n, s->Y, T, s->dY, s->dYt, ld, s->loss_part, s->bias_part);
-    if ((rc = check_launch("loss_grad_kernel")) < 0) return rc;
-    // backward data: G3 = (dY W4) * [H3 > 0], G2 = (G3 W3) * [H2 > 0], G1 = (G2 W2) * [H1 > 0]; each
-    // epilogue also writes its tiles' column sums (the bias gradients' partials)
-    GemmArgs g = nt(s->dY, kOutPad, s->W4t, kOutPad, n, kHid, kOutPad);
-    g.epi = kEpiMask; g.H = s->H3; g.ldh = kHid; g.Cb = s->G3; g.ldc = kHid; g.Ct = s->G3t; g.ldt = ld;
-    g.bias_part = s->bias_part; g.bias_col = kOut;
-    if ((rc = gemm(g, 1, st)) < 0) return rc;
-    g = nt(s->G3, kHid, s->W3t, kHid, n, kHid, kHid);
-    g.epi = kEpiMask; g.H = s->H2; g.ldh = kHid; g.Cb = s->G2; g.ldc = kHid; g.Ct = s->G2t; g.ldt = ld;
-    g.bias_part = s->bias_part; g.bias_col = kOut + kHid;
-    if ((rc = gemm(g, 1, st)) < 0) return rc;
-    g = nt(s->G2, kHid, s->W2t, kHid, n, kHid, kHid);
-    g.epi = kEpiMask; g.H = s->H1; g.ldh = kHid; g.Cb = nullptr; g.Ct = s->G1t; g.ldt = ld;
-    g.bias_part = s->bias_part; g.bias_col = kOut + 2 * kHid;
-    if ((rc = gemm(g, 1, st)) < 0) return rc;
-    // weight gradients (the batch is the K dimension), each layer's partials in its own region
-    const size_t r3 = kGradCount[0], r2 = r3 + kGradCount[1], r1 = r2 + kGradCount[2];
-    if ((rc = weight_grad(s, n, s->dYt, kOut, s->H3t, kHid, 0, st)) < 0) return rc;
-    if ((rc = weight_grad(s, n, s->G3t, kHid, s->H2t, kHid, r3, st)) < 0) return rc;
-    if ((rc = weight_grad(s, n, s->G2t, kHid, s->H1t, kHid, r2, st)) < 0) return rc;
-    // W1's product is [128 x 32]; the reduction keeps the 22 real inputs
-    if ((rc = weight_grad(s, n, s->G1t, kHid, s->Xt, kInPad, r1, st)) < 0) return rc;
-    const int splits = (n + split_len(n) - 1) / split_len(n);
-    hipLaunchKernelGGL(grad_reduce_kernel, dim3((kGradTotal + kBiasCols + kReduceLanes - 1) / kReduceLanes), dim3(256), 0, st, splits, blocks,
-                       (n + kTile - 1) / kTile, s->part, s->bias_part, s->grads);
-    if ((rc = check_launch("grad_reduce_kernel")) < 0) return rc;
-    if (loss_host) {
-        std::vector<float> lp(static_cast<size_t>(blocks));
-        if (hipMemcpyAsync(lp.data(), s->loss_part, lp.size() * sizeof(float), hipMemcpyDeviceToHost, st) != hipSuccess ||
-            hipStreamSynchronize(st) != hipSuccess)
-            return set_error(PLT_EHIP, "plt_surrogate: loss read-back failed");
-        double sum = 0.0;
-        for (float v : lp) sum += v;
-        *loss_host = float(sum / (double(n) * kOut));
-    }
-    return PLT_OK;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -815,14 +539,6 @@ __global__ void __launch_bounds__(kEw) prep_targets_kernel(int n, const float* _
     for (int k = 0; k < kOut; ++k) T[size_t(i) * kOut + k] = float((y[k] - dstat[k]) / dstat[kOut + k]);
 }
 
-// Device-side state of plt_surrogate_train: every launch of a training step reads what it needs
-// from here, so one captured step replays as every step.
-struct TrainState {
-    uint32_t step, steps_per_epoch, steps_total, batch, n_valid, seed, adam_t;
-    float lr0;
-};
-static_assert(sizeof(TrainState) <= kTrainStateWords * 4, "train state size");
-
 __host__ __device__ inline uint32_t mix32(uint32_t h) {
     h ^= h >> 16;
     h *= 0x7FEB352Du;
@@ -865,91 +581,446 @@ __global__ void shuffle_kernel(uint32_t n, int half, uint32_t key, uint32_t* __r
     if (x < n) out[x] = shuffle_index(x, n, half, key);
 }
 
-// One training batch: row i is the valid sample idx[shuffle(pos)] of this epoch's order, packed
-// as the bf16 inputs (both layouts) and the FP32 targets.
-__global__ void __launch_bounds__(kEw) gather_pack_kernel(const TrainState* __restrict__ st, const uint32_t* __restrict__ idx,
-                                                          const float* __restrict__ X, const float* __restrict__ T, __bf16* __restrict__ Xb,
-                                                          __bf16* __restrict__ Xt, int ldt, float* __restrict__ Tb, int half) {
-    const TrainState s = *st;
-    const uint32_t i = blockIdx.x * kEw + threadIdx.x;
-    if (i >= s.batch) return;
-    const uint32_t epoch = s.step / s.steps_per_epoch;
-    const uint32_t pos = (s.step % s.steps_per_epoch) * s.batch + i;
-    const uint32_t j = idx[shuffle_index(pos, s.n_valid, half, epoch_key(s.seed, epoch))];
+// ---------------------------------------------------------------------------------------
+// Fused training step: forward pass, loss, backward pass and the weight gradients of one batch in
+// one kernel. A workgroup of four waves takes every gridDim.x-th tile of 64 samples; a tile's
+// activations never leave LDS, and the gradients of all 38,032 parameters are summed over the
+// group's tiles in its waves' accumulators (176 registers a lane) and written once, as one partial
+// per group. grad_reduce_kernel sums the partials in group order (and, in training, applies Adam), so
+// a step is two launches.
+//
+// Products are computed transposed as in mlp_infer_kernel (weights the A operand, out[feature x
+// sample]); wave w holds features 32w..32w+31. Each activation and each back-propagated gradient is
+// stored twice: sample-major rows (the next product's B operand: 8 consecutive features) and
+// feature-major rows (the weight gradients contract over samples, so both their operands are 8
+// consecutive samples of one feature). A hidden unit's ReLU mask is one bit in the lane that
+// computed it, which is the lane that computes its gradient.
+//
+// It is bound by the chain of ten barriers per tile with one group per CU (125 KB of LDS): a batch of
+// 16,384 is 256 tiles over 128 groups. Before, a step was eighteen dependent launches (a GEMM per
+// product and gradient, 9 us each, every activation through memory in two layouts): 141 us.
+// ---------------------------------------------------------------------------------------
+constexpr int kGroupsMax = 128;  // partials to sum: more groups write and read more of them (20 MB at 128)
+constexpr int kTRow = kFTile + 8;  // feature-major LDS rows
+
+// The layout of one group's partial: W4, W3, W2, W1 (its 32 padded inputs), then the biases b4, b3, b2, b1.
+constexpr int kPartW4 = 0, kPartW3 = kPartW4 + kOut * kHid, kPartW2 = kPartW3 + kHid * kHid, kPartW1 = kPartW2 + kHid * kHid,
+              kGradTotal = kPartW1 + kHid * kInPad;  // 38,912
+constexpr int kBiasCols = kOut + 3 * kHid;
+constexpr int kPartTotal = kGradTotal + kBiasCols;
+
+// Device-side state of plt_surrogate_train: every launch of a training step reads what it needs
+// from here, so one captured step replays as every step. The train kernel reads `step` and publishes
+// the step it runs, its learning rate and Adam's corrections (group 0); the reduction reads those and
+// advances `step`.
+struct TrainState {
+    uint32_t step, steps_per_epoch, steps_total, batch, n_valid, seed, adam_t0;
+    float lr0;
+    uint32_t now;
+    float lr, c1, c2;
+};
+
+struct TrainArgs {
+    int n;                 // rows of the batch
+    const float *X, *T;    // inputs [. x 22] and targets [. x 16]
+    const uint32_t* idx;   // with st: row i of the batch is idx[shuffle(step's i-th position)]
+    int half;
+    TrainState* st;
+    const __bf16 *W1, *W2, *W3, *W4, *W2t, *W3t, *W4t;
+    const float *b1, *b2, *b3, *b4;
+    float* part;           // [gridDim.x x kPartTotal]
+    float* loss_part;      // [gridDim.x]
+};
+
+__global__ void __launch_bounds__(kFThreads, 1) mlp_train_kernel(TrainArgs g) {
+    __shared__ __bf16 xs[kFTile * kXRow], xt[kInPad * kTRow];
+    __shared__ __bf16 sa[kFTile * kHRow], sb[kFTile * kHRow];          // sample-major, ping-pong
+    __shared__ __bf16 h1t[kHid * kTRow], h2t[kHid * kTRow], h3t[kHid * kTRow], gt[kHid * kTRow];
+    __shared__ __bf16 dy[kFTile * kXRow], dyt[kOut * kTRow];
+    __shared__ uint32_t rows[kFTile];
+    __shared__ float red[kFThreads / 64][1 + kOut];
+    const int t = threadIdx.x, w = t >> 6, lane = t & 63;
+    const int fr = lane & 15, fg = lane >> 4, fk = 8 * fg;
+    uint32_t step = 0, epoch_pos = 0, key = 0, n_valid = 0;
+    if (g.st) {
+        const TrainState s = *g.st;
+        step = s.step;
+        n_valid = s.n_valid;
+        epoch_pos = (step % s.steps_per_epoch) * s.batch;
+        key = epoch_key(s.seed, step / s.steps_per_epoch);
+        if (blockIdx.x == 0 && t == 0) {
+            // the cosine-decayed rate (at least 1e-6) and the corrections of Adam step adam_t0 + step + 1
+            const double tt = double(s.adam_t0) + double(step) + 1.0;
+            g.st->now = step;
+            g.st->c1 = float(1.0 - pow(double(0.9f), tt));
+            g.st->c2 = float(1.0 - pow(double(0.999f), tt));
+            const double cs = cos(3.14159265358979323846 * double(step) / double(max(1u, s.steps_total)));
+            g.st->lr = float(fmax(double(s.lr0) * 0.5 * (1.0 + cs), 1e-6));
+        }
+    }
+    // outputs 16..31 of dY pad its K dimension with zeros
+    for (int i = t; i < kFTile * kXRow; i += kFThreads) dy[i] = static_cast<__bf16>(0.f);
+    f32x4 c1[2], c2[2], c3[2], c4;
 #pragma unroll
-    for (int f = 0; f < kInPad; ++f) {
-        const __bf16 v = static_cast<__bf16>(f < kIn ? X[size_t(j) * kIn + f] : 0.f);
-        Xb[size_t(i) * kInPad + f] = v;
-        Xt[size_t(f) * ldt + i] = v;
+    for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int f = 32 * w + 16 * cb + 4 * fg + r;
+            c1[cb][r] = g.b1[f];
+            c2[cb][r] = g.b2[f];
+            c3[cb][r] = g.b3[f];
+        }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) c4[r] = g.b4[4 * fg + r];
+    const f32x4 zero{0.f, 0.f, 0.f, 0.f};
+    f32x4 dw1[2][2], dw2[2][8], dw3[2][8], dw4[2], db1[2], db2[2], db3[2], db4 = zero;
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+#pragma unroll
+        for (int b = 0; b < 8; ++b) dw2[a][b] = dw3[a][b] = zero;
+        dw1[a][0] = dw1[a][1] = dw4[a] = db1[a] = db2[a] = db3[a] = zero;
+    }
+    float loss = 0.f;
+    const float scale = 2.f / (float(g.n) * float(kOut));
+
+    // out[32w..32w+31 x 64 samples] from kb blocks of 32 sample-major inputs and the weight rows Wm
+    auto product = [&](auto kblocks, const __bf16* in, int in_row, const __bf16* Wm, int ldw, const f32x4* init, f32x4 (&acc)[2][4]) {
+        constexpr int kK = decltype(kblocks)::value;
+        bf16x8 wf[2][kK];
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+            for (int kb = 0; kb < kK; ++kb)
+                wf[cb][kb] = *reinterpret_cast<const bf16x8*>(Wm + size_t(32 * w + 16 * cb + fr) * ldw + 32 * kb + fk);
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) acc[cb][s] = init ? init[cb] : zero;
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int kb = 0; kb < kK; ++kb) {
+                const bf16x8 b = *reinterpret_cast<const bf16x8*>(in + (16 * s + fr) * in_row + 32 * kb + fk);
+#pragma unroll
+                for (int cb = 0; cb < 2; ++cb) acc[cb][s] = mfma(wf[cb][kb], b, acc[cb][s]);
+            }
+    };
+    // stores a lane's four features of sample 16 s + fr in both layouts (sm may be null)
+    auto store = [&](bf16x4 h, int cb, int s, __bf16* sm, __bf16* fm) {
+        const int f = 32 * w + 16 * cb + 4 * fg, row = 16 * s + fr;
+        if (sm) *reinterpret_cast<bf16x4*>(sm + row * kHRow + f) = h;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) fm[(f + r) * kTRow + row] = h[r];
+    };
+    auto forward = [&](auto kblocks, const __bf16* in, int in_row, const __bf16* Wm, int ldw, const f32x4* bias, __bf16* sm, __bf16* fm) {
+        f32x4 acc[2][4];
+        product(kblocks, in, in_row, Wm, ldw, bias, acc);
+        uint32_t mask = 0;
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                bf16x4 h;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    h[r] = static_cast<__bf16>(relu_bits(acc[cb][s][r]));
+                    mask |= static_cast<float>(h[r]) > 0.f ? 1u << (16 * cb + 4 * s + r) : 0u;
+                }
+                store(h, cb, s, sm, fm);
+            }
+        return mask;
+    };
+    auto backward = [&](auto kblocks, const __bf16* in, int in_row, const __bf16* Wt, int ldw, uint32_t mask, __bf16* sm, __bf16* fm, f32x4 (&db)[2]) {
+        f32x4 acc[2][4];
+        product(kblocks, in, in_row, Wt, ldw, nullptr, acc);
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                bf16x4 h;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    h[r] = static_cast<__bf16>((mask >> (16 * cb + 4 * s + r)) & 1u ? acc[cb][s][r] : 0.f);
+                    db[cb][r] += static_cast<float>(h[r]);
+                }
+                store(h, cb, s, sm, fm);
+            }
+    };
+    // dW[32w..32w+31 x 16 B..] += G H^T over the tile's 64 samples (feature-major operands)
+    auto weight_grad = [&](auto nb, const __bf16* gm, const __bf16* hm, auto& dw) {
+        constexpr int kB = decltype(nb)::value;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            bf16x8 a[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) a[i] = *reinterpret_cast<const bf16x8*>(gm + (32 * w + 16 * i + fr) * kTRow + 32 * kb + fk);
+#pragma unroll
+            for (int b = 0; b < kB; ++b) {
+                const bf16x8 h = *reinterpret_cast<const bf16x8*>(hm + (16 * b + fr) * kTRow + 32 * kb + fk);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) dw[i][b] = mfma(a[i], h, dw[i][b]);
+            }
+        }
+    };
+    using K1 = std::integral_constant<int, 1>;
+    using K2 = std::integral_constant<int, 2>;
+    using K4 = std::integral_constant<int, 4>;
+    using K8 = std::integral_constant<int, 8>;
+
+    const int ntiles = (g.n + kFTile - 1) / kFTile;
+    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        const int r0 = tile * kFTile;
+        __syncthreads();  // the previous tile's last reads of xt, gt and rows
+        if (t < kFTile) {
+            uint32_t row = uint32_t(min(r0 + t, g.n - 1));
+            if (g.st) row = g.idx[shuffle_index(epoch_pos + row, n_valid, g.half, key)];
+            rows[t] = row;
+        }
+        __syncthreads();
+        {
+            // thread t stages input features 2p, 2p + 1 (p = t % 16) of rows t / 16 + 16 j; rows past n
+            // and padding features are zero
+            const int p = t & 15, sr = t >> 4;
+            const bool in = 2 * p < kIn;
+            float2 v[kFTile / 16];
+#pragma unroll
+            for (int j = 0; j < kFTile / 16; ++j)
+                v[j] = *reinterpret_cast<const float2*>(g.X + size_t(rows[sr + 16 * j]) * kIn + (in ? 2 * p : 0));
+#pragma unroll
+            for (int j = 0; j < kFTile / 16; ++j) {
+                const int r = sr + 16 * j;
+                const bool live = in && r0 + r < g.n;
+                bf16x2 pv;
+                pv[0] = static_cast<__bf16>(live ? v[j].x : 0.f);
+                pv[1] = static_cast<__bf16>(live ? v[j].y : 0.f);
+                *reinterpret_cast<bf16x2*>(xs + r * kXRow + 2 * p) = pv;
+                xt[(2 * p) * kTRow + r] = pv[0];
+                xt[(2 * p + 1) * kTRow + r] = pv[1];
+            }
+        }
+        // the lane's four targets: outputs 4 fg.. of sample 16 w + fr
+        const int srow = 16 * w + fr;
+        const f32x4 target = *reinterpret_cast<const f32x4*>(g.T + size_t(rows[srow]) * kOut + 4 * fg);
+        __syncthreads();
+        const uint32_t m1 = forward(K1{}, xs, kXRow, g.W1, kInPad, c1, sa, h1t);
+        __syncthreads();
+        const uint32_t m2 = forward(K4{}, sa, kHRow, g.W2, kHid, c2, sb, h2t);
+        __syncthreads();
+        const uint32_t m3 = forward(K4{}, sb, kHRow, g.W3, kHid, c3, sa, h3t);
+        __syncthreads();
+        {
+            f32x4 y = c4;
+#pragma unroll
+            for (int kb = 0; kb < 4; ++kb)
+                y = mfma(*reinterpret_cast<const bf16x8*>(g.W4 + size_t(fr) * kHid + 32 * kb + fk),
+                         *reinterpret_cast<const bf16x8*>(sa + srow * kHRow + 32 * kb + fk), y);
+            const bool live = r0 + srow < g.n;
+            bf16x4 d;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float e = live ? y[r] - target[r] : 0.f;
+                loss += e * e;
+                d[r] = static_cast<__bf16>(scale * e);
+                db4[r] += static_cast<float>(d[r]);
+                dyt[(4 * fg + r) * kTRow + srow] = d[r];
+            }
+            *reinterpret_cast<bf16x4*>(dy + srow * kXRow + 4 * fg) = d;
+        }
+        __syncthreads();
+        backward(K1{}, dy, kXRow, g.W4t, kOutPad, m3, sb, gt, db3);
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {  // dW4[16 x 32w..32w+31]
+            const bf16x8 a = *reinterpret_cast<const bf16x8*>(dyt + fr * kTRow + 32 * kb + fk);
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+                dw4[b] = mfma(a, *reinterpret_cast<const bf16x8*>(h3t + (32 * w + 16 * b + fr) * kTRow + 32 * kb + fk), dw4[b]);
+        }
+        __syncthreads();
+        weight_grad(K8{}, gt, h2t, dw3);
+        backward(K4{}, sb, kHRow, g.W3t, kHid, m2, sa, h3t, db2);  // h3t now holds the second layer's gradient
+        __syncthreads();
+        weight_grad(K8{}, h3t, h1t, dw2);
+        backward(K4{}, sa, kHRow, g.W2t, kHid, m1, static_cast<__bf16*>(nullptr), gt, db1);
+        __syncthreads();
+        weight_grad(K2{}, gt, xt, dw1);
+    }
+    // the group's partial. D layout: the lane holds rows 4 fg + r of column fr of each 16 x 16 block
+    float* part = g.part + size_t(blockIdx.x) * kPartTotal;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int o = 32 * w + 16 * i + 4 * fg + r;
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+                part[kPartW3 + o * kHid + 16 * b + fr] = dw3[i][b][r];
+                part[kPartW2 + o * kHid + 16 * b + fr] = dw2[i][b][r];
+            }
+#pragma unroll
+            for (int b = 0; b < 2; ++b) part[kPartW1 + o * kInPad + 16 * b + fr] = dw1[i][b][r];
+            part[kPartW4 + (4 * fg + r) * kHid + 32 * w + 16 * i + fr] = dw4[i][r];
+        }
+    // bias sums over the 16 lanes of a feature (xor steps 1..8), in a fixed order
+    auto lanes16 = [](float v) {
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) v += __shfl_xor(v, o);
+        return v;
+    };
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int f = 32 * w + 16 * i + 4 * fg + r;
+            const float s3 = lanes16(db3[i][r]), s2 = lanes16(db2[i][r]), s1 = lanes16(db1[i][r]);
+            if (fr == 0) {
+                part[kGradTotal + kOut + f] = s3;
+                part[kGradTotal + kOut + kHid + f] = s2;
+                part[kGradTotal + kOut + 2 * kHid + f] = s1;
+            }
+        }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const float s = lanes16(db4[r]);
+        if (fr == 0) red[w][1 + 4 * fg + r] = s;
     }
 #pragma unroll
-    for (int f = 0; f < kOut; ++f) Tb[size_t(i) * kOut + f] = T[size_t(j) * kOut + f];
+    for (int o = 1; o < 64; o <<= 1) loss += __shfl_xor(loss, o);
+    if (lane == 0) red[w][0] = loss;
+    __syncthreads();
+    if (t <= kOut) {
+        const float s = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
+        if (t == 0) g.loss_part[blockIdx.x] = s;
+        else part[kGradTotal + t - 1] = s;
+    }
 }
+static_assert(sizeof(TrainState) <= kTrainStateWords * 4, "train state size");
 
-// The bf16 operand copies of the four weight matrices (W [out x in_pad], Wt [in x out_pad]).
+// Every gradient from the groups' partials, in one launch. A block takes 64 elements of a partial
+// with four threads each: thread group q sums the partials of groups q, q + 4, ... (16 loads issued
+// before their adds), and the four sums are combined in order. The sum goes to `grads`, or (grads
+// null) through Adam to the FP32 master parameters and their bf16 copies, whose padding stays zero;
+// the learning rate and the corrections come from the arguments, or with `st` from the device state
+// that the train kernel published. Block 0 then also records the step's mean loss and advances the
+// state's step, which no thread of this kernel reads.
 struct WeightCopies {
     __bf16 *W1, *W1t, *W2, *W2t, *W3, *W3t, *W4, *W4t;
 };
-
-// Adam on the FP32 master parameters fused with the bf16 copies of each updated weight (the
-// padding of the copies stays zero). The learning rate and the bias corrections come from the
-// arguments, or with `st` from the device state: the cosine-decayed rate lr0 (1 + cos(pi step /
-// steps)) / 2 (at least 1e-6) and the corrections of Adam step adam_t + 1.
-__global__ void adam_cast_kernel(int count, float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                                 float* __restrict__ v, const TrainState* __restrict__ st, float lr, float c1, float c2, float b1, float b2,
-                                 float eps, WeightCopies w) {
-    const int e = blockIdx.x * kEw + threadIdx.x;
-    if (e >= count) return;
-    if (st) {
-        const TrainState s = *st;
-        const double tt = double(s.adam_t) + 1.0;
-        c1 = float(1.0 - pow(double(b1), tt));
-        c2 = float(1.0 - pow(double(b2), tt));
-        const double cs = cos(3.14159265358979323846 * double(s.step) / double(max(1u, s.steps_total)));
-        lr = float(fmax(double(s.lr0) * 0.5 * (1.0 + cs), 1e-6));
+struct ReduceArgs {
+    int groups;
+    const float *part, *loss_part;
+    float* grads;
+    float *p, *m, *v;
+    TrainState* st;
+    float lr, c1, c2;
+    WeightCopies w;
+    float* loss_hist;
+};
+constexpr int kReduceLanes = 64, kReduceBatch = 16;  // elements per block; loads in flight per thread
+__global__ void __launch_bounds__(256) grad_reduce_kernel(ReduceArgs a) {
+    __shared__ float sums[4][kReduceLanes];
+    const int el = threadIdx.x & (kReduceLanes - 1), q = threadIdx.x >> 6;
+    const int e = blockIdx.x * kReduceLanes + el;
+    const bool live = e < kPartTotal;
+    float acc = 0.f;
+    if (live) {
+        for (int z0 = q; z0 < a.groups; z0 += 4 * kReduceBatch) {
+            float v[kReduceBatch];
+#pragma unroll
+            for (int j = 0; j < kReduceBatch; ++j) {
+                const int z = z0 + 4 * j;
+                v[j] = z < a.groups ? a.part[size_t(z) * kPartTotal + e] : 0.f;
+            }
+#pragma unroll
+            for (int j = 0; j < kReduceBatch; ++j) acc += v[j];
+        }
     }
-    const float ge = g[e];
-    const float me = b1 * m[e] + (1.f - b1) * ge;
-    const float ve = b2 * v[e] + (1.f - b2) * ge * ge;
-    m[e] = me;
-    v[e] = ve;
-    const float pe = p[e] - lr * (me / c1) / (sqrtf(ve / c2) + eps);
-    p[e] = pe;
-    const __bf16 h = static_cast<__bf16>(pe);
-    if (size_t(e) < kOffB1) {
-        const int o = e / kIn, i = e % kIn;
-        w.W1[o * kInPad + i] = h;
-        w.W1t[i * kHid + o] = h;
-    } else if (size_t(e) >= kOffW2 && size_t(e) < kOffB2) {
-        const int l = int(e - kOffW2), o = l / kHid, i = l % kHid;
-        w.W2[o * kHid + i] = h;
-        w.W2t[i * kHid + o] = h;
-    } else if (size_t(e) >= kOffW3 && size_t(e) < kOffB3) {
-        const int l = int(e - kOffW3), o = l / kHid, i = l % kHid;
-        w.W3[o * kHid + i] = h;
-        w.W3t[i * kHid + o] = h;
-    } else if (size_t(e) >= kOffW4 && size_t(e) < kOffB4) {
-        const int l = int(e - kOffW4), o = l / kHid, i = l % kHid;
-        w.W4[o * kHid + i] = h;
-        w.W4t[i * kOutPad + o] = h;
+    sums[q][el] = acc;
+    __syncthreads();
+    if (a.st && blockIdx.x == 0 && q == 1) {
+        double l = 0.0;
+        for (int z = el; z < a.groups; z += kReduceLanes) l += double(a.loss_part[z]);
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) l += __shfl_xor(l, o);
+        if (el == 0) {
+            const uint32_t now = a.st->now;
+            a.loss_hist[now] = float(l / (double(a.st->batch) * kOut));
+            a.st->step = now + 1u;
+        }
+    }
+    if (q != 0 || !live) return;
+    const float ge = (sums[0][el] + sums[1][el]) + (sums[2][el] + sums[3][el]);
+    // the element's parameter and, for a weight, its places in the two bf16 copies
+    size_t dst;
+    __bf16 *W = nullptr, *Wt = nullptr;
+    if (e < kPartW3) {
+        const int o = e / kHid, i = e % kHid;
+        dst = kOffW4 + e;
+        W = a.w.W4 + e;
+        Wt = a.w.W4t + i * kOutPad + o;
+    } else if (e < kPartW1) {
+        const bool third = e < kPartW2;
+        const int l = e - (third ? kPartW3 : kPartW2), o = l / kHid, i = l % kHid;
+        dst = (third ? kOffW3 : kOffW2) + l;
+        W = (third ? a.w.W3 : a.w.W2) + l;
+        Wt = (third ? a.w.W3t : a.w.W2t) + i * kHid + o;
+    } else if (e < kGradTotal) {
+        const int l = e - kPartW1, o = l / kInPad, i = l % kInPad;
+        if (i >= kIn) return;  // padding
+        dst = kOffW1 + size_t(o) * kIn + i;
+        W = a.w.W1 + l;
+        Wt = a.w.W1t + i * kHid + o;
+    } else {
+        const int c = e - kGradTotal;
+        dst = c < kOut ? kOffB4 + c : c < kOut + kHid ? kOffB3 + (c - kOut) : c < kOut + 2 * kHid ? kOffB2 + (c - kOut - kHid)
+                                                                                      : kOffB1 + (c - kOut - 2 * kHid);
+    }
+    if (a.grads) {
+        a.grads[dst] = ge;
+        return;
+    }
+    constexpr float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+    const float lr = a.st ? a.st->lr : a.lr, c1 = a.st ? a.st->c1 : a.c1, c2 = a.st ? a.st->c2 : a.c2;
+    const float me = b1 * a.m[dst] + (1.f - b1) * ge;
+    const float ve = b2 * a.v[dst] + (1.f - b2) * ge * ge;
+    a.m[dst] = me;
+    a.v[dst] = ve;
+    const float pe = a.p[dst] - lr * (me / c1) / (sqrtf(ve / c2) + eps);
+    a.p[dst] = pe;
+    if (W) {
+        const __bf16 h = static_cast<__bf16>(pe);
+        *W = h;
+        *Wt = h;
     }
 }
 WeightCopies weight_copies(const plt_surrogate* s) { return WeightCopies{s->W1, s->W1t, s->W2, s->W2t, s->W3, s->W3t, s->W4, s->W4t}; }
 
-// End of a step: its mean loss (the loss kernel's block partials, summed in order) and the counters.
-__global__ void step_end_kernel(TrainState* __restrict__ st, const float* __restrict__ loss_part, int blocks, float* __restrict__ loss_hist) {
-    if (threadIdx.x != 0) return;
-    double acc = 0.0;
-    for (int b = 0; b < blocks; ++b) acc += double(loss_part[b]);
-    loss_hist[st->step] = float(acc / (double(st->batch) * kOut));
-    st->step += 1u;
-    st->adam_t += 1u;
+int train_groups(uint32_t n) { return int(std::min<uint32_t>(kGroupsMax, (n + kFTile - 1) / kFTile)); }
+
+// The two launches of a step over n rows of X and T (with `st`, rows idx[shuffle]): the partials, then
+// their sums into `grads` or through Adam.
+int train_launch(plt_surrogate* s, int n, const float* X, const float* T, const uint32_t* idx, int half, TrainState* st, float* grads, float lr,
+                 float c1, float c2, float* loss_hist, hipStream_t qs) {
+    const int groups = train_groups(uint32_t(n));
+    const TrainArgs ta{n, X, T, idx, half, st, s->W1, s->W2, s->W3, s->W4, s->W2t, s->W3t, s->W4t,
+                       s->params + kOffB1, s->params + kOffB2, s->params + kOffB3, s->params + kOffB4, s->part, s->loss_part};
+    hipLaunchKernelGGL(mlp_train_kernel, dim3(groups), dim3(kFThreads), 0, qs, ta);
+    int rc = check_launch("mlp_train_kernel");
+    if (rc < 0) return rc;
+    const ReduceArgs ra{groups, s->part, s->loss_part, grads, s->params, s->adam_m, s->adam_v, st, lr, c1, c2, weight_copies(s), loss_hist};
+    hipLaunchKernelGGL(grad_reduce_kernel, dim3((kPartTotal + kReduceLanes - 1) / kReduceLanes), dim3(256), 0, qs, ra);
+    return check_launch("grad_reduce_kernel");
 }
 
-int pack(plt_surrogate* s, int n, const float* X, bool with_t, hipStream_t st) {
-    const int ld = int(s->max_batch);
-    hipLaunchKernelGGL(pack_inputs_kernel, dim3((n + kEw - 1) / kEw), dim3(kEw), 0, st, n, X, s->Xb, with_t ? s->Xt : nullptr, ld);
-    return check_launch("pack_inputs_kernel");
+// The mean loss of the last train_launch over n rows.
+int read_loss(plt_surrogate* s, uint32_t n, float* loss, hipStream_t st) {
+    std::vector<float> lp(static_cast<size_t>(train_groups(n)));
+    if (hipMemcpyAsync(lp.data(), s->loss_part, lp.size() * sizeof(float), hipMemcpyDeviceToHost, st) != hipSuccess ||
+        hipStreamSynchronize(st) != hipSuccess)
+        return set_error(PLT_EHIP, "plt_surrogate: loss read-back failed");
+    double sum = 0.0;
+    for (float v : lp) sum += v;
+    *loss = float(sum / (double(n) * kOut));
+    return PLT_OK;
 }
 
 }  // namespace
@@ -986,7 +1057,6 @@ int plt_surrogate_create(plt_context* ctx, uint32_t max_batch, uint32_t seed, pl
     auto* s = new plt_surrogate;
     s->ctx = ctx;
     s->max_batch = max_batch;
-    const size_t B = max_batch;
     int rc = PLT_OK;
     auto A = [&](auto** p, size_t count) { if (rc == PLT_OK) rc = dev_alloc(s, p, count); };
     A(&s->params, kParams); A(&s->grads, kParams); A(&s->adam_m, kParams); A(&s->adam_v, kParams);
@@ -994,24 +1064,12 @@ int plt_surrogate_create(plt_context* ctx, uint32_t max_batch, uint32_t seed, pl
     A(&s->W2, size_t(kHid) * kHid); A(&s->W2t, size_t(kHid) * kHid);
     A(&s->W3, size_t(kHid) * kHid); A(&s->W3t, size_t(kHid) * kHid);
     A(&s->W4, size_t(kOut) * kHid); A(&s->W4t, size_t(kHid) * kOutPad);
-    A(&s->Xb, B * kInPad); A(&s->Xt, B * kInPad);
-    A(&s->H1, B * kHid); A(&s->H1t, B * kHid); A(&s->H2, B * kHid); A(&s->H2t, B * kHid); A(&s->H3, B * kHid); A(&s->H3t, B * kHid);
-    A(&s->dY, B * kOutPad); A(&s->dYt, B * kOut);
-    A(&s->G3, B * kHid); A(&s->G3t, B * kHid); A(&s->G2, B * kHid); A(&s->G2t, B * kHid); A(&s->G1t, B * kHid);
-    A(&s->Y, B * kOut);
-    A(&s->part, size_t(kSplitTarget) * kGradTotal);
-    A(&s->loss_part, (B + kEw - 1) / kEw);
-    A(&s->bias_part, (B / kTile + 1) * size_t(kBiasCols));
+    A(&s->part, size_t(train_groups(max_batch)) * kPartTotal);
+    A(&s->loss_part, size_t(train_groups(max_batch)));
     A(&s->train_state, kTrainStateWords);
     A(&s->stats, 2 * kOut + 2 * kIn);
     A(&s->counter, 1);
     if (rc != PLT_OK) { plt_surrogate_destroy(s); return rc; }
-    // the batch (K) padding of every feature-major operand must read as zeros
-    const size_t tbytes = B * kHid * sizeof(__bf16);
-    for (__bf16* p : {s->H1t, s->H2t, s->H3t, s->G3t, s->G2t, s->G1t})
-        if (hipMemset(p, 0, tbytes) != hipSuccess) rc = set_error(PLT_EHIP, "plt_surrogate_create: clear failed");
-    if (hipMemset(s->dYt, 0, B * kOut * sizeof(__bf16)) != hipSuccess || hipMemset(s->Xt, 0, B * kInPad * sizeof(__bf16)) != hipSuccess)
-        rc = set_error(PLT_EHIP, "plt_surrogate_create: clear failed");
     // He-uniform initialisation of the weights (bound sqrt(6 / fan_in)), zero biases
     std::vector<float> p(kParams, 0.f);
     std::mt19937 gen(seed);
@@ -1069,8 +1127,8 @@ int plt_surrogate_gradients(plt_surrogate* s, uint32_t n, const float* X, const 
         return set_error(PLT_EINVAL, "plt_surrogate_gradients: bad arguments (n a multiple of 32, at most max_batch)");
     const hipStream_t st = static_cast<hipStream_t>(stream);
     int rc;
-    if ((rc = pack(s, int(n), X, true, st)) < 0) return rc;
-    if ((rc = loss_and_grads(s, int(n), T, loss, st)) < 0) return rc;
+    if ((rc = train_launch(s, int(n), X, T, nullptr, 0, nullptr, s->grads, 0.f, 1.f, 1.f, nullptr, st)) < 0) return rc;
+    if (loss && (rc = read_loss(s, n, loss, st)) < 0) return rc;
     if (grads_host) {
         if (hipMemcpyAsync(grads_host, s->grads, kParams * sizeof(float), hipMemcpyDeviceToHost, st) != hipSuccess ||
             hipStreamSynchronize(st) != hipSuccess)
@@ -1083,15 +1141,12 @@ int plt_surrogate_train_step(plt_surrogate* s, uint32_t n, const float* X, const
     if (!s || n == 0 || n % 32 || n > s->max_batch || !X || !T || !(lr > 0.f))
         return set_error(PLT_EINVAL, "plt_surrogate_train_step: bad arguments (n a multiple of 32, at most max_batch)");
     const hipStream_t st = static_cast<hipStream_t>(stream);
-    int rc;
-    if ((rc = pack(s, int(n), X, true, st)) < 0) return rc;
-    if ((rc = loss_and_grads(s, int(n), T, loss, st)) < 0) return rc;
-    ++s->step;
     const float b1 = 0.9f, b2 = 0.999f;
-    const float c1 = 1.f - std::pow(b1, float(s->step)), c2 = 1.f - std::pow(b2, float(s->step));
-    hipLaunchKernelGGL(adam_cast_kernel, dim3((kParams + kEw - 1) / kEw), dim3(kEw), 0, st, kParams, s->params, s->grads, s->adam_m,
-                       s->adam_v, nullptr, lr, c1, c2, b1, b2, 1e-8f, weight_copies(s));
-    return check_launch("adam_cast_kernel");
+    const float k = float(s->step + 1), c1 = 1.f - std::pow(b1, k), c2 = 1.f - std::pow(b2, k);
+    int rc;
+    if ((rc = train_launch(s, int(n), X, T, nullptr, 0, nullptr, nullptr, lr, c1, c2, nullptr, st)) < 0) return rc;
+    ++s->step;
+    return loss ? read_loss(s, n, loss, st) : PLT_OK;
 }
 
 int plt_surrogate_prepare(plt_surrogate* s, uint32_t n, const float* X, const float* M, float* T, uint32_t* idx, uint32_t* n_valid,
@@ -1156,28 +1211,16 @@ int plt_surrogate_train(plt_surrogate* s, uint32_t n_valid, const uint32_t* idx,
     if (total >= (uint64_t(1) << 31)) return set_error(PLT_EINVAL, "plt_surrogate_train: too many steps");
     const int half = shuffle_half(n_valid);
     const hipStream_t st = static_cast<hipStream_t>(stream);
-    const TrainState ts{0u, spe, uint32_t(total), batch, n_valid, seed, s->step, lr};
-    // the step's own buffers: the batch's targets and the per-step losses
-    void* q = nullptr;
-    if (hipMalloc(&q, size_t(batch) * kOut * 4 + size_t(total) * 4) != hipSuccess)
-        return set_error(PLT_ENOMEM, "plt_surrogate_train: buffer allocation failed");
-    float* Tb = static_cast<float*>(q);
-    float* loss_hist = Tb + size_t(batch) * kOut;
-    const int lblocks = int((batch + kEw - 1) / kEw);
+    const TrainState ts{0u, spe, uint32_t(total), batch, n_valid, seed, s->step, lr, 0u, lr, 1.f, 1.f};
+    void* q = nullptr;  // the per-step losses
+    if (hipMalloc(&q, size_t(total) * 4) != hipSuccess) return set_error(PLT_ENOMEM, "plt_surrogate_train: buffer allocation failed");
+    float* loss_hist = static_cast<float*>(q);
     auto* state = reinterpret_cast<TrainState*>(s->train_state);
     int rc = PLT_OK;
     if (hipMemcpyAsync(state, &ts, sizeof(ts), hipMemcpyHostToDevice, st) != hipSuccess || hipStreamSynchronize(st) != hipSuccess)
         rc = set_error(PLT_EHIP, "plt_surrogate_train: state upload failed");
     auto step = [&](hipStream_t qs) -> int {
-        hipLaunchKernelGGL(gather_pack_kernel, dim3(lblocks), dim3(kEw), 0, qs, state, idx, X, T, s->Xb, s->Xt, int(s->max_batch), Tb, half);
-        int r;
-        if ((r = check_launch("gather_pack_kernel")) < 0) return r;
-        if ((r = loss_and_grads(s, int(batch), Tb, nullptr, qs)) < 0) return r;
-        hipLaunchKernelGGL(adam_cast_kernel, dim3((kParams + kEw - 1) / kEw), dim3(kEw), 0, qs, kParams, s->params, s->grads, s->adam_m,
-                           s->adam_v, state, 0.f, 1.f, 1.f, 0.9f, 0.999f, 1e-8f, weight_copies(s));
-        if ((r = check_launch("adam_cast_kernel")) < 0) return r;
-        hipLaunchKernelGGL(step_end_kernel, dim3(1), dim3(64), 0, qs, state, s->loss_part, lblocks, loss_hist);
-        return check_launch("step_end_kernel");
+        return train_launch(s, int(batch), X, T, idx, half, state, nullptr, 0.f, 1.f, 1.f, loss_hist, qs);
     };
     if (rc == PLT_OK && graph) {
         // one step captured and replayed: every step-dependent value is in the device state
@@ -1221,9 +1264,7 @@ int plt_surrogate_train(plt_surrogate* s, uint32_t n_valid, const uint32_t* idx,
 // Raw GEMM (C = A * Bt^T, bf16 operands, FP32 output) for tests of the matrix-core kernel.
 int plt_mlp_gemm_nt(uint32_t M, uint32_t N, uint32_t K, const void* A, const void* Bt, float* C, plt_stream stream) {
     if (!A || !Bt || !C) return set_error(PLT_EINVAL, "plt_mlp_gemm_nt: bad arguments");
-    GemmArgs g = nt(static_cast<const __bf16*>(A), int(K), static_cast<const __bf16*>(Bt), int(K), int(M), int(N), int(K));
-    g.epi = kEpiF32; g.Cf = C; g.ldc = int(N);
-    return gemm(g, 1, static_cast<hipStream_t>(stream));
+    return gemm(GemmArgs{static_cast<const __bf16*>(A), static_cast<const __bf16*>(Bt), int(M), int(N), int(K), C}, static_cast<hipStream_t>(stream));
 }
 
 }  // extern "C"

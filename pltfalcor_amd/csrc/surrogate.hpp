@@ -13,11 +13,7 @@ struct plt_surrogate {
     uint32_t step = 0;
     // bf16 operands: W (row-major [out x in_pad]) and Wt ([in x out_pad]) per layer
     __bf16 *W1 = nullptr, *W1t = nullptr, *W2 = nullptr, *W2t = nullptr, *W3 = nullptr, *W3t = nullptr, *W4 = nullptr, *W4t = nullptr;
-    // activations: sample-major and feature-major (ld = max_batch) copies
-    __bf16 *Xb = nullptr, *Xt = nullptr, *H1 = nullptr, *H1t = nullptr, *H2 = nullptr, *H2t = nullptr, *H3 = nullptr, *H3t = nullptr;
-    __bf16 *dY = nullptr, *dYt = nullptr, *G3 = nullptr, *G3t = nullptr, *G2 = nullptr, *G2t = nullptr, *G1t = nullptr;
-    float *Y = nullptr, *part = nullptr, *loss_part = nullptr;
-    float* bias_part = nullptr;       // bias-gradient partials per batch tile
+    float *part = nullptr, *loss_part = nullptr;  // a training step's gradient and loss partials, one per workgroup
     uint32_t* train_state = nullptr;  // device-side training step state (plt_surrogate_train)
     // target statistics and the inputs' training box (plt_surrogate_set_stats): 16 + 16 + 22 + 22
     float* stats = nullptr;

@@ -383,3 +383,76 @@ def test_gpu_surrogate_graph_training_equals_eager(gpu):
         assert np.array_equal(np.sort(o), np.arange(n))
         orders.append(o)
     assert (orders[0] != orders[1]).mean() > 0.9
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [32, 64, 96, 4128, 8256])
+def test_gpu_surrogate_fused_step_at_tile_edges(gpu, n):
+    """Loss and gradients of batches around the training kernel's 64-row tiles (half a tile, one, one
+    and a half) and its 128 workgroups (65 tiles; 129, so one group takes two) against the restatement
+    with the same bf16 roundings. A sum in another order changes a result by FP32 rounding, or flips the
+    bf16 rounding of an activation (a relative 2^-9 of it): 1e-3 of a tensor's norm allows a quarter of
+    its activations to flip."""
+    import torch
+    from pltfalcor_amd.surrogate import Surrogate
+    ctx, _ = _ctx_with_drude()
+    s = Surrogate(ctx, max_batch=n, seed=5)
+    p = R.he_init(n).astype(np.float32)
+    s.set_params(p)
+    rng = np.random.default_rng(n)
+    X = rng.uniform(-1, 1, (n, 22)).astype(np.float32)
+    T = rng.normal(0, 1, (n, 16)).astype(np.float32)
+    g, loss = s.gradients(torch.tensor(X, device="cuda"), torch.tensor(T, device="cuda"))
+    lr, gr = R.loss_and_grad(p.astype(np.float64), X.astype(np.float64), T.astype(np.float64), R.bf16)
+    assert abs(loss - lr) <= 1e-5 * lr
+    o = 0
+    for name, shape in R.SHAPES:
+        k = int(np.prod(shape))
+        a, b = g[o:o + k], gr[o:o + k]
+        err = np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-30)
+        print(f"n {n} {name}: {err:.2e}")
+        assert err <= 1e-3, name
+        o += k
+    s.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch", [96, 2048])
+def test_gpu_surrogate_train_equals_steps_on_the_shuffled_rows(gpu, batch):
+    """plt_surrogate_train gathers each batch in its kernel: the same as train_step on the rows that
+    plt_surrogate_shuffle lists, at the cosine-decayed rates. Adam's bias corrections are single
+    precision there and double here (c2 = 1 - 0.999^t loses up to 1e-4 of itself to cancellation, half
+    of that reaches a step of at most about lr per parameter)."""
+    import ctypes as C
+    import torch
+    from pltfalcor_amd import _lib
+    from pltfalcor_amd.surrogate import ExactSamples, Surrogate, prepare
+    ctx, _ = _ctx_with_drude()
+    S = ExactSamples(ctx, 3 * batch + 40, seed=12)
+    lib, lr, steps = _lib.load(), 2e-3, 2
+    runs = []
+    for fused in (True, False):
+        s = Surrogate(ctx, max_batch=batch, seed=2)
+        T, idx, nv = prepare(s, S)
+        n = steps * batch + 7
+        assert nv >= n
+        if fused:
+            losses = np.zeros(1, np.float32)
+            _lib.check(lib.plt_surrogate_train(s.handle, n, C.c_void_p(idx.data_ptr()), C.c_void_p(S.X.data_ptr()),
+                                               C.c_void_p(T.data_ptr()), batch, 1, lr, 9, 1,
+                                               losses.ctypes.data_as(C.POINTER(C.c_float)), None))
+        else:
+            order = torch.empty(n, dtype=torch.int32, device="cuda")
+            _lib.check(lib.plt_surrogate_shuffle(n, 9, 0, C.c_void_p(order.data_ptr()), None))
+            got = []
+            for k in range(steps):
+                rows = idx[order[k * batch:(k + 1) * batch].long()].long()
+                got.append(s.train_step(S.X[rows].contiguous(), T[rows].contiguous(),
+                                        lr * 0.5 * (1 + np.cos(np.pi * k / steps)), want_loss=True))
+            losses = np.array([np.mean(got)], np.float32)
+        runs.append((s.get_params(), losses[0]))
+        s.close()
+    d = np.abs(runs[0][0] - runs[1][0]).max()
+    print(f"batch {batch}: largest parameter difference {d:.2e}")
+    assert d <= 1e-4 * lr * steps + 1e-7
+    assert abs(runs[0][1] - runs[1][1]) <= 1e-5 * runs[1][1]

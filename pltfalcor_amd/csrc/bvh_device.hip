@@ -507,23 +507,15 @@ uint32_t build_top(std::vector<TopCluster>& c, size_t b, size_t e, int depth, ui
     return id;
 }
 
-// Device allocations of one build, released together unless kept.
-struct Allocs {
-    std::vector<void*> ptrs;
-    ~Allocs() {
-        for (void* p : ptrs)
-            if (p) (void)hipFree(p);
-    }
+// Carves the build's arrays out of one allocation (base null: only adds up the size).
+struct Carve {
+    char* base;
+    size_t used = 0;
     template <typename T>
     T* get(size_t count) {
-        void* p = nullptr;
-        if (hipMalloc(&p, count * sizeof(T) > 0 ? count * sizeof(T) : 16) != hipSuccess) return nullptr;
-        ptrs.push_back(p);
-        return static_cast<T*>(p);
-    }
-    void keep(void* p) {
-        for (void*& q : ptrs)
-            if (q == p) q = nullptr;
+        T* p = reinterpret_cast<T*>(base + used);
+        used += (count * sizeof(T) + 255) & ~size_t(255);
+        return p;
     }
 };
 
@@ -536,41 +528,79 @@ inline unsigned grid_of(uint32_t n) { return (n + kBlock - 1) / kBlock; }
 
 }  // namespace
 
-int build_bvh_device(const DeviceSceneBuffers& d, hipStream_t st, DeviceBvh& out) {
+void BvhWork::release() {
+    for (void* p : {scratch, static_cast<void*>(nodes), static_cast<void*>(tris)})
+        if (p) (void)hipFree(p);
+    *this = BvhWork{};
+}
+
+// The scratch arrays and the tree's own buffers come from `work`. Allocated and freed by each build,
+// as twenty allocations of up to 670 MB, they took longer than the build: rebuilding the tree of
+// 5.24 M triangles and casting a million rays took 54 ms (14 ms for a scene's first rebuild), of which
+// the kernels are 7.5 ms.
+int build_bvh_device(const DeviceSceneBuffers& d, hipStream_t st, BvhWork& work, DeviceBvh& out) {
     const uint32_t n = d.n_tris;
     if (n == 0) return set_error(PLT_EINVAL, "device BVH build: the scene has no triangles");
     // leaf references hold (first << 3) | (count - 1) in 31 bits
     if (n >= (1u << 28)) return set_error(PLT_EINVAL, "device BVH build: more than 2^28 triangles");
     const auto t0 = std::chrono::steady_clock::now();
-    Allocs A;
     const size_t nn2 = 2 * size_t(n);
     const uint32_t box_blocks = grid_of(n) < kBoxBlocks ? grid_of(n) : kBoxBlocks;
-    uint32_t* words = A.get<uint32_t>(8);  // [7]: the next level's width
-    float* cb = A.get<float>(6);
-    float* partial = A.get<float>(6 * size_t(box_blocks));
-    float4* tlo = A.get<float4>(n);  // triangle boxes, later the second cluster list
-    float4* thi = A.get<float4>(n);
-    uint64_t* bufA = A.get<uint64_t>(n);  // keys, then flags, then collapse items
-    uint64_t* bufB = A.get<uint64_t>(n);  // sorted keys, then scanned flags, then next items
-    uint32_t* vals = A.get<uint32_t>(n);
-    uint32_t* ids = A.get<uint32_t>(n);
-    float4* nlo = A.get<float4>(nn2);
-    float4* nhi = A.get<float4>(nn2);
-    uint32_t* ncnt = A.get<uint32_t>(nn2);
-    float4* clo = A.get<float4>(n);
-    float4* chi = A.get<float4>(n);
-    uint32_t* nn = A.get<uint32_t>(n);
-    float4* nodes = A.get<float4>(8 * size_t(n));
-    float4* tris = A.get<float4>(3 * size_t(n));
-    if (!words || !cb || !partial || !tlo || !thi || !bufA || !bufB || !vals || !ids || !nlo || !nhi || !ncnt || !clo || !chi || !nn || !nodes || !tris)
-        return set_error(PLT_ENOMEM, "device BVH build: hipMalloc failed");
     size_t sort_bytes = 0, scan_bytes = 0;
-    if (rocprim::radix_sort_pairs(nullptr, sort_bytes, bufA, bufB, vals, ids, n, 0, 63, st) != hipSuccess ||
-        rocprim::inclusive_scan(nullptr, scan_bytes, bufA, bufB, size_t(n), rocprim::plus<uint64_t>(), st) != hipSuccess)
+    if (rocprim::radix_sort_pairs(nullptr, sort_bytes, static_cast<uint64_t*>(nullptr), static_cast<uint64_t*>(nullptr),
+                                  static_cast<uint32_t*>(nullptr), static_cast<uint32_t*>(nullptr), n, 0, 63, st) != hipSuccess ||
+        rocprim::inclusive_scan(nullptr, scan_bytes, static_cast<uint64_t*>(nullptr), static_cast<uint64_t*>(nullptr), size_t(n),
+                                rocprim::plus<uint64_t>(), st) != hipSuccess)
         return hip_fail("temporary storage query");
-    void* tmp = A.get<uint8_t>(sort_bytes > scan_bytes ? sort_bytes : scan_bytes);
-    if (!tmp) return set_error(PLT_ENOMEM, "device BVH build: hipMalloc failed");
     const size_t tmp_bytes = sort_bytes > scan_bytes ? sort_bytes : scan_bytes;
+    uint32_t *words, *vals, *ids, *ncnt, *nn;
+    float *cb, *partial;
+    float4 *tlo, *thi, *nlo, *nhi, *clo, *chi, *nodes;
+    uint64_t *bufA, *bufB;
+    void* tmp;
+    auto carve = [&](char* base) {
+        Carve c{base};
+        words = c.get<uint32_t>(8);  // [7]: the next level's width
+        cb = c.get<float>(6);
+        partial = c.get<float>(6 * size_t(box_blocks));
+        tlo = c.get<float4>(n);  // triangle boxes, later the second cluster list
+        thi = c.get<float4>(n);
+        bufA = c.get<uint64_t>(n);  // keys, then flags, then collapse items
+        bufB = c.get<uint64_t>(n);  // sorted keys, then scanned flags, then next items
+        vals = c.get<uint32_t>(n);
+        ids = c.get<uint32_t>(n);
+        nlo = c.get<float4>(nn2);
+        nhi = c.get<float4>(nn2);
+        ncnt = c.get<uint32_t>(nn2);
+        clo = c.get<float4>(n);
+        chi = c.get<float4>(n);
+        nn = c.get<uint32_t>(n);
+        nodes = c.get<float4>(8 * size_t(n));
+        tmp = c.get<uint8_t>(tmp_bytes);
+        return c.used;
+    };
+    const size_t need = carve(nullptr);
+    if (need > work.scratch_bytes) {
+        if (work.scratch) (void)hipFree(work.scratch);
+        work.scratch = nullptr;
+        work.scratch_bytes = 0;
+        if (hipMalloc(&work.scratch, need) != hipSuccess) {
+            work.scratch = nullptr;
+            (void)hipGetLastError();
+            return set_error(PLT_ENOMEM, "device BVH build: hipMalloc failed");
+        }
+        work.scratch_bytes = need;
+    }
+    (void)carve(static_cast<char*>(work.scratch));
+    if (!work.tris) {
+        void* p = nullptr;
+        if (hipMalloc(&p, 3 * size_t(n) * sizeof(float4)) != hipSuccess) {
+            (void)hipGetLastError();
+            return set_error(PLT_ENOMEM, "device BVH build: hipMalloc failed");
+        }
+        work.tris = static_cast<float4*>(p);
+    }
+    float4* tris = work.tris;
 
     hipLaunchKernelGGL(tri_box_kernel, dim3(box_blocks), dim3(kBlock), 0, st, n, d.positions, d.indices, tlo, thi, partial);
     hipLaunchKernelGGL(bounds_kernel, dim3(1), dim3(kBlock), 0, st, box_blocks, partial, cb);
@@ -665,10 +695,21 @@ int build_bvh_device(const DeviceSceneBuffers& d, hipStream_t st, DeviceBvh& out
         std::swap(items, next);
         ++levels;
     }
-    // depth-first layout, into an allocation of the exact size (the clustering's counts and
+    // depth-first layout, into a buffer of its own (the clustering's counts and
     // neighbour lists are free again: sizes in ncnt, positions in nn, both at least n_nodes long)
-    float4* exact = A.get<float4>(8 * size_t(level_base));
-    if (!exact) return set_error(PLT_ENOMEM, "device BVH build: hipMalloc failed");
+    if (level_base > work.nodes_cap) {
+        if (work.nodes) (void)hipFree(work.nodes);
+        work.nodes = nullptr;
+        work.nodes_cap = 0;
+        void* p = nullptr;
+        if (hipMalloc(&p, 8 * size_t(level_base) * sizeof(float4)) != hipSuccess) {
+            (void)hipGetLastError();
+            return set_error(PLT_ENOMEM, "device BVH build: hipMalloc failed");
+        }
+        work.nodes = static_cast<float4*>(p);
+        work.nodes_cap = level_base;
+    }
+    float4* exact = work.nodes;
     uint32_t* size = ncnt;
     uint32_t* at = nn;
     for (int l = levels - 1; l >= 0; --l)
@@ -680,11 +721,12 @@ int build_bvh_device(const DeviceSceneBuffers& d, hipStream_t st, DeviceBvh& out
                            level_width[l], nodes, size, at);
     hipLaunchKernelGGL(permute_kernel, dim3(grid_of(level_base)), dim3(kBlock), 0, st, level_base, nodes, at, exact);
     if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) return hip_fail("layout");
-    A.keep(exact);
-    A.keep(tris);
     out.nodes = exact;
     out.tris = tris;
     out.n_nodes = level_base;
+    out.nodes_cap = work.nodes_cap;
+    work.nodes = work.tris = nullptr;  // the caller's now
+    work.nodes_cap = 0;
     out.max_depth = levels;
     out.iterations = iterations;
     out.ms = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - t0).count();

@@ -99,6 +99,7 @@ int upload_bvh(const HostScene& hs, DeviceSceneBuffers& d) {
     d.tris = dt;
     d.n_tris = uint32_t(nt);
     d.n_nodes = uint32_t(hs.bvh.nodes.size());
+    d.nodes_cap = hs.bvh.nodes.size();
     return PLT_OK;
 }
 
@@ -129,18 +130,32 @@ void host_bvh_info(const HostScene& hs, plt_bvh_info& info) {
     info.build_ms = hs.bvh.build_ms;
 }
 
-// Builds the scene's tree on the device and installs it; the scene keeps its old tree on failure.
+// Builds the scene's tree on the device and installs it; the scene keeps its old tree on failure. The
+// old tree's buffers go to the scene's build workspace.
 int device_bvh(plt_scene* s, hipStream_t st) {
     DeviceBvh b;
-    const int rc = build_bvh_device(s->dev, st, b);
+    const int rc = build_bvh_device(s->dev, st, s->work, b);
     if (rc < 0) return rc;
     if (hipDeviceSynchronize() != hipSuccess) {
         (void)hipFree(b.nodes);
         (void)hipFree(b.tris);
         return set_error(PLT_EHIP, "device BVH build: device synchronization failed");
     }
-    replace_owned(s->dev, s->dev.nodes, b.nodes);
-    replace_owned(s->dev, s->dev.tris, b.tris);
+    auto swap_owned = [&](float4* old, float4* now) {  // false: the scene held none
+        for (void*& p : s->dev.owned)
+            if (old && p == old) {
+                p = now;
+                return true;
+            }
+        s->dev.owned.push_back(now);
+        return false;
+    };
+    if (swap_owned(s->dev.nodes, b.nodes)) {
+        s->work.nodes = s->dev.nodes;
+        s->work.nodes_cap = s->dev.nodes_cap;
+    }
+    if (swap_owned(s->dev.tris, b.tris)) s->work.tris = s->dev.tris;
+    s->dev.nodes_cap = b.nodes_cap;
     s->dev.nodes = b.nodes;
     s->dev.tris = b.tris;
     s->dev.n_nodes = b.n_nodes;
@@ -238,6 +253,7 @@ int plt_scene_create_ex(plt_context* ctx, const plt_scene_desc* d, int builder, 
     if (builder == PLT_BVH_DEVICE_PLOC) {
         rc = plt::upload_arrays(h, s->dev);
         if (rc >= 0) rc = plt::device_bvh(s, nullptr);
+        s->work.release();  // most scenes are built once
         if (rc == PLT_EINVAL) {  // too deep for the traversal stack: the host builder bounds the depth
             h.bvh = plt::build_bvh(h.positions, h.indices, 4);
             plt::host_bvh_info(h, s->bvh);
@@ -345,6 +361,7 @@ int plt_scene_set_camera(plt_scene* scene, const plt_camera* camera) {
 int plt_scene_destroy(plt_scene* scene) {
     if (!scene) return PLT_OK;
     plt::free_scene(scene->dev);
+    scene->work.release();
     delete scene;
     return PLT_OK;
 }

@@ -288,3 +288,21 @@ def test_gpu_render_identical_with_either_tree(gpu):
     valid = np.arange(r0.shape[0])[:, None] < L[None, :]  # records past a path's end are not written
     assert np.array_equal(r0.transpose(0, 2, 1)[valid], r1.transpose(0, 2, 1)[valid])
     assert np.array_equal(c0, c1) and np.array_equal(a0, a1) and np.array_equal(n0, n1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [5, 3000])
+def test_gpu_rebuilds_reuse_the_scenes_buffers(gpu, n):
+    """A scene's device rebuilds alternate between two trees' buffers and one scratch area: every
+    rebuild, also across host rebuilds (whose buffers have another size), gives a well-formed tree that
+    casts like brute force."""
+    from pltfalcor_amd.bsdf import Context
+    print(f"rebuilds n={n}", flush=True)
+    ctx = Context(0)
+    a, base, pos, nrm, idx = _soup(n, seed=n + 1)
+    s = _from(ctx, a, base, pos, nrm, idx, "device")
+    for builder in ("device", "device", "host", "device", "device", "host", "host", "device"):
+        assert s.build_bvh(builder)["builder"] == builder
+        nodes, tris = s.bvh_arrays()
+        check_tree(nodes, tris, pos, idx)
+        _trace_both(s, pos, idx, random_rays(1000, n, lo=-12, hi=12))

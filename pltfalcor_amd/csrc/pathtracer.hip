@@ -261,25 +261,23 @@ int launch_solve_pass_split(const PtScene& sc, const PtFrame& fr, const SolveBuf
     if (after_light) (void)hipEventRecord(after_light, st);
     // manifold walks: only frames with manifold NEE queue any, but the kernel is cheap to launch
     // empty and a captured graph then holds the same launches whatever the options
-    if (surrogate || !fork.aux) {
+    if (surrogate) {
         if ((rc = launch_solve_walks(sc, fr, sb, st)) < 0) return rc;
         if (after_walk) (void)hipEventRecord(after_walk, st);
-        if ((rc = surrogate ? launch_solve_unwind_surrogate(sc, fr, sb, surrogate, st) : launch_solve_unwind(sc, fr, sb, st)) < 0)
-            return rc;
+        if ((rc = launch_solve_unwind_surrogate(sc, fr, sb, surrogate, st)) < 0) return rc;
     } else {
-        // The walk kernel's last walks keep a few waves busy for milliseconds: the events that are
+        // The walk kernel's last walks keep a few waves busy for long: the events that are
         // not walks are unwound beside it on the second stream (their contributions stored), the
         // walks that succeeded after it, and then every path's contributions are summed in order.
-        SolveBuffers staged = sb;
-        staged.stage = 1u;
-        if (hipEventRecord(fork.fork, st) != hipSuccess || hipStreamWaitEvent(fork.aux, fork.fork, 0) != hipSuccess)
+        const hipStream_t side = fork.aux ? fork.aux : st;
+        if (fork.aux && (hipEventRecord(fork.fork, st) != hipSuccess || hipStreamWaitEvent(fork.aux, fork.fork, 0) != hipSuccess))
             return set_error(PLT_EHIP, "split solve pass: fork to the second stream failed");
-        if ((rc = launch_solve_unwind(sc, fr, staged, fork.aux)) < 0) return rc;
-        if (hipEventRecord(fork.join, fork.aux) != hipSuccess) return set_error(PLT_EHIP, "split solve pass: join event failed");
+        if ((rc = launch_solve_unwind(sc, fr, sb, side)) < 0) return rc;
+        if (fork.aux && hipEventRecord(fork.join, fork.aux) != hipSuccess) return set_error(PLT_EHIP, "split solve pass: join event failed");
         if ((rc = launch_solve_walks(sc, fr, sb, st)) < 0) return rc;
         if (after_walk) (void)hipEventRecord(after_walk, st);
         if ((rc = launch_solve_walk_unwind(sc, fr, sb, st)) < 0) return rc;
-        if (hipStreamWaitEvent(st, fork.join, 0) != hipSuccess) return set_error(PLT_EHIP, "split solve pass: join failed");
+        if (fork.aux && hipStreamWaitEvent(st, fork.join, 0) != hipSuccess) return set_error(PLT_EHIP, "split solve pass: join failed");
         if ((rc = launch_solve_sum(fr, sb, st)) < 0) return rc;
     }
     if (after_unwind) (void)hipEventRecord(after_unwind, st);

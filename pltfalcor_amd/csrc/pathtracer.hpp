@@ -112,7 +112,9 @@ __host__ __device__ inline uint32_t path_pixel(uint32_t width, uint32_t height, 
 // path's own vertex order. Walk vertices of manifold NEE events live in a second area, kHitWords
 // planes per vertex, 64 * hits_per_path per region.
 enum EvField {
-    kEvMeta = 0,  // lane (6 bits) | vertex (7 bits) << 6 | kind (2 bits) << 13 | kEvBit* | walk vertices << 21
+    // lane (6 bits) | vertex (7 bits) << 6 | kind (2 bits) << 13 | kEvBit* | walk vertices (4 bits) << 21 |
+    // material type of the vertex (4 bits) << kEvTypeShift
+    kEvMeta = 0,
     kEvLe,        // 4 planes: sourced spectral radiance per HWSS component
     kEvLam = kEvLe + 4,  // 4 planes: wavelengths
     kEvPos = kEvLam + 4, // 3 planes: beam position (area sources)
@@ -133,6 +135,7 @@ enum : uint32_t {
     kEvBitComps1 = 1u << 15, kEvBitDistant = 1u << 16, kEvBitMnee = 1u << 17, kEvBitMisL = 1u << 18,
     kEvBitCurrentMs = 1u << 19, kEvBitDispersive = 1u << 20
 };
+constexpr uint32_t kEvTypeShift = 25;
 enum HitField { kHitTri = 0, kHitB1, kHitB2, kHitPos, kHitLobe = kHitPos + 3, kHitWords };
 constexpr uint32_t kSolveRegion = 64;  // paths per region: one wave of the split solve kernels
 constexpr size_t kEventsPerExecute = 6;  // kernel-timing events per execute of the pass
@@ -170,12 +173,10 @@ struct SolveBuffers {
     uint32_t ev_per_path, hits_per_path;
     size_t ev_cap, hit_cap;  // plane lengths: regions * 64 * per-path capacity
     WalkQueue walk;
-    // Staged unwind: the unwind kernel with `stage` set writes the RGB contribution of every event
-    // that is not a manifold walk into `contrib` (3 planes of ev_cap) and sums nothing; the
-    // walk-unwind kernel adds the walks' contributions, and the sum kernel adds each path's
-    // contributions in slot order (the megakernel's order) and writes the colour.
+    // Staged unwind: the staged unwind kernel writes the RGB contribution of every event that is not a
+    // manifold walk (3 planes of ev_cap), the walk-unwind kernel adds the walks', and the sum kernel
+    // adds each path's contributions in slot order (the megakernel's order) and writes the colour.
     float* contrib;
-    uint32_t stage;
     SurPath sur;             // used by the query and apply unwind modes only
 };
 

@@ -158,6 +158,7 @@ solve_sample_kernel(PtScene sc, PtFrame fr, SolveBuffers sb) {
             const Surf s = surface_at(sc, bounce.tri, bounce.b1, bounce.b2, bounce.wi);
             const Mat m = material_at(sc, s.material);
             const uint32_t props = mat_props(m);
+            const uint32_t typeBits = (m.type & 15u) << kEvTypeShift;
 
             // ---- NEE (pltpt_solve.rt.slang:245-366) up to the beam's transport ----
             if (doNEE) {
@@ -333,7 +334,7 @@ solve_sample_kernel(PtScene sc, PtFrame fr, SolveBuffers sb) {
                             }
                             size_t e;
                             if (!reserve(e)) break;
-                            uint32_t meta = metaBase | (kEvKindNee << 13) | compsBit | (bDistant ? kEvBitDistant : 0u) |
+                            uint32_t meta = metaBase | (kEvKindNee << 13) | compsBit | typeBits | (bDistant ? kEvBitDistant : 0u) |
                                             (misL ? kEvBitMisL : 0u);
                             if (mnee)
                                 meta |= kEvBitMnee | (currentVertexMS ? kEvBitCurrentMs : 0u) | (ms.dispersive ? kEvBitDispersive : 0u) |
@@ -400,7 +401,7 @@ solve_sample_kernel(PtScene sc, PtFrame fr, SolveBuffers sb) {
                     const float dist = sqrtf(dot(dd, dd));
                     size_t e;
                     if (!reserve(e)) break;
-                    ev_put(sb, e, kEvMeta, metaBase | (kEvKindEmissive << 13) | compsBit);
+                    ev_put(sb, e, kEvMeta, metaBase | (kEvKindEmissive << 13) | compsBit | typeBits);
                     ev_put_source<N>(sb, e, Le, lam, s.pos, bounce.wi, fr.sourcing_area, dist);
                 }
             }
@@ -700,15 +701,151 @@ struct PathSums {
     }
 };
 
+// The exact unwind kernels write the contribution of every event, one lane per event; events do not
+// depend on each other, so any grouping will do. A region holds about 22 events: a wave per region left
+// two thirds of its lanes idle, and the active ones spent each step in up to ten materials' code one
+// after the other and waited for the longest path (9 of 64 lanes active on average). So a block of four
+// waves takes many events together and orders them by a counting sort in LDS: by the number of steps,
+// the longest first, so that a block does not end on them, then by the material of the vertex that the
+// light sample was taken at, which for half of the events is the only step. Its waves then take 64
+// events at a time (fewer when the block has few, so that all four have work), mostly of one kind.
+//
 // Two waves per SIMD: the beam, the material instance and the evaluation temporaries fit the 256
-// registers without spilling, and this kernel (no traversal, few dependent fetches) loses less to
-// the lower occupancy than it gains (1080p depth 8: 1.30 ms per frame at two waves, 2.14 ms at four
-// with 612 B of scratch per lane, 2.59 ms at six). Mode: exact unwind, or the surrogate's query or
-// apply pass (the query pass writes no colour). With sb.stage set (exact mode) it writes the
-// contributions of the events that are not manifold walks and sums nothing.
+// registers without spilling. 1280 x 720 without walks: 0.61 -> 0.40 ms for 474,000 events (0.56 at
+// three waves per SIMD, with the shortest first 0.51, and 0.74 with neighbouring regions in one block).
+constexpr int kUnwindBlock = 256, kUnwindRegions = 64, kUnwindBins = 128;
+constexpr uint32_t kUnwindList = 4096;  // events sorted at a time
+struct UnwindShared {
+    uint32_t bins[kUnwindBins + 1];
+    uint32_t list[kUnwindList];
+    uint32_t taken;
+};
+// `steps` - 1 and the material type as a sort key below kUnwindBins.
+PLT_DEV uint32_t unwind_key(uint32_t steps, uint32_t meta) { return ((7u - min(steps - 1u, 7u)) << 4) | ((meta >> kEvTypeShift) & 15u); }
+
+// Unwinds the block's events event_of(0 .. total - 1) whose key_of is below kUnwindBins. Every thread of
+// the block calls it, with the same total.
+template <int N, class EventOf, class KeyOf>
+PLT_DEV void unwind_sorted(const PtScene& sc, const PtFrame& fr, const SolveBuffers& sb, UnwindShared& sh, uint32_t total, EventOf&& event_of,
+                           KeyOf&& key_of) {
+    const uint32_t t = threadIdx.x, lane = t & 63u;
+    const size_t regionEvents = size_t(kPtBlock) * sb.ev_per_path;
+    for (uint32_t base = 0; base < total; base += kUnwindList) {
+        const uint32_t m = min(total - base, kUnwindList);
+        if (t <= uint32_t(kUnwindBins)) sh.bins[t] = 0u;
+        __syncthreads();
+        for (uint32_t i = t; i < m; i += kUnwindBlock) {
+            const uint32_t k = key_of(event_of(base + i));
+            if (k < uint32_t(kUnwindBins)) atomicAdd(&sh.bins[k], 1u);
+        }
+        __syncthreads();
+        if (t < 64u) {  // exclusive scan of the bins, two per lane; bins[kUnwindBins] becomes their sum
+            const uint32_t c0 = sh.bins[2 * lane], c1 = sh.bins[2 * lane + 1];
+            uint32_t s = c0 + c1;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const uint32_t v = __shfl_up(s, o);
+                s += int(lane) >= o ? v : 0u;
+            }
+            sh.bins[2 * lane] = s - c1 - c0;
+            sh.bins[2 * lane + 1] = s - c1;
+            if (lane == 63u) sh.bins[kUnwindBins] = s;
+            if (lane == 0u) sh.taken = 0u;
+        }
+        __syncthreads();
+        const uint32_t count = sh.bins[kUnwindBins];
+        for (uint32_t i = t; i < m; i += kUnwindBlock) {
+            const uint32_t e = event_of(base + i), k = key_of(e);
+            if (k < uint32_t(kUnwindBins)) sh.list[atomicAdd(&sh.bins[k], 1u)] = e;
+        }
+        __syncthreads();
+        // the waves take `chunk` events at a time; every wave leaves once the list is used up
+        const uint32_t chunk = max(16u, min(64u, (count + 3u) / 4u));
+        for (;;) {
+            uint32_t k = 0;
+            if (lane == 0u) k = atomicAdd(&sh.taken, chunk);
+            k = uint32_t(__builtin_amdgcn_readfirstlane(int(k)));
+            if (k >= count) break;
+            if (lane < chunk && k + lane < count) {
+                const size_t e = sh.list[k + lane];
+                float c[3] = {0.f, 0.f, 0.f};
+                unwind_event<N, kUnwindExact>(sc, fr, sb, e, ev_get(sb, e, kEvMeta), uint32_t(e / regionEvents), c);
+                contrib_put(sb, e, c);
+            }
+        }
+        __syncthreads();  // the list and the bins are rewritten
+    }
+}
+// Whether the event belongs to a path that is left to the megakernel.
+PLT_DEV bool path_overflowed(const SolveBuffers& sb, uint32_t e, uint32_t meta) {
+    const uint32_t* rg = sb.region + size_t(e / (size_t(kPtBlock) * sb.ev_per_path)) * kRegWords;
+    const uint32_t who = meta & 63u;
+    return ((rg[who < 32u ? kRegOverflowLo : kRegOverflowHi] >> (who & 31u)) & 1u) != 0u;
+}
+
+// The events that are not manifold walks, beside the walk kernel: a block takes regions blockIdx.x,
+// + gridDim.x, ... (at most kUnwindRegions), so that neighbouring regions (sky, or a dense object) go to
+// different blocks and blocks get about as many events each. The walk kernel may turn a walk's event void
+// between the two passes of the sort; neither kind is unwound here.
+template <int N>
+__global__ void __launch_bounds__(kUnwindBlock) __attribute__((amdgpu_waves_per_eu(2, 2)))
+solve_unwind_staged_kernel(PtScene sc, PtFrame fr, SolveBuffers sb, uint32_t regions) {
+    __shared__ UnwindShared sh;
+    __shared__ uint32_t first[kUnwindRegions + 1];  // running event count before each region of the block
+    const uint32_t t = threadIdx.x, lane = t & 63u;
+    const uint32_t nr = (regions - blockIdx.x + gridDim.x - 1u) / gridDim.x;
+    const size_t regionEvents = size_t(kPtBlock) * sb.ev_per_path;
+    if (t < 64u) {  // the first wave: inclusive scan of the regions' counts
+        uint32_t c = lane < nr ? sb.region[size_t(blockIdx.x + lane * gridDim.x) * kRegWords + kRegEvents] : 0u;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t v = __shfl_up(c, o);
+            c += int(lane) >= o ? v : 0u;
+        }
+        first[lane + 1] = c;
+        if (lane == 0) first[0] = 0u;
+    }
+    __syncthreads();
+    unwind_sorted<N>(
+        sc, fr, sb, sh, first[kUnwindRegions],
+        [&](uint32_t g) {
+            uint32_t lo = 0, hi = nr - 1;  // the last region that starts at or before g
+            while (lo < hi) {
+                const uint32_t mid = (lo + hi + 1) / 2;
+                if (first[mid] <= g) lo = mid;
+                else hi = mid - 1;
+            }
+            return uint32_t(size_t(blockIdx.x + lo * gridDim.x) * regionEvents + (g - first[lo]));
+        },
+        [&](uint32_t e) {
+            const uint32_t meta = sb.ev[size_t(kEvMeta) * sb.ev_cap + e];
+            if (((meta >> 13) & 3u) == kEvKindVoid || is_walk_event(meta) || path_overflowed(sb, e, meta)) return uint32_t(kUnwindBins);
+            return unwind_key(1u + ((meta >> 6) & 127u), meta);
+        });
+}
+
+// After the walk kernel: the walks that succeeded (the void ones add nothing), from the walk queue.
+template <int N>
+__global__ void __launch_bounds__(kUnwindBlock) __attribute__((amdgpu_waves_per_eu(2, 2)))
+solve_walk_unwind_kernel(PtScene sc, PtFrame fr, SolveBuffers sb) {
+    __shared__ UnwindShared sh;
+    const uint32_t queued = sb.walk.counters[0];
+    const uint32_t mine = queued > blockIdx.x ? (queued - blockIdx.x + gridDim.x - 1u) / gridDim.x : 0u;
+    unwind_sorted<N>(
+        sc, fr, sb, sh, mine, [&](uint32_t g) { return sb.walk.items[blockIdx.x + g * gridDim.x]; },
+        [&](uint32_t e) {
+            const uint32_t meta = sb.ev[size_t(kEvMeta) * sb.ev_cap + e];
+            if (((meta >> 13) & 3u) == kEvKindVoid || path_overflowed(sb, e, meta)) return uint32_t(kUnwindBins);
+            return unwind_key(1u + ((meta >> 6) & 127u) + ((meta >> 21) & 15u), meta);
+        });
+}
+
+// The surrogate's query and apply passes (the query pass writes no colour), a wave per region, which
+// also sums each path's contributions in slot order, the order the megakernel adds them in.
 template <int N, int Mode>
 __global__ void __launch_bounds__(kPtBlock) __attribute__((amdgpu_waves_per_eu(2, 2)))
 solve_unwind_kernel(PtScene sc, PtFrame fr, SolveBuffers sb) {
+    static_assert(Mode == kUnwindQuery || Mode == kUnwindApply, "the exact unwind is solve_unwind_staged_kernel");
     __shared__ float part[3][kPtBlock];
     __shared__ uint32_t owner[kPtBlock];
     const uint32_t lane = threadIdx.x, region = blockIdx.x;
@@ -716,7 +853,6 @@ solve_unwind_kernel(PtScene sc, PtFrame fr, SolveBuffers sb) {
     const uint32_t count = rg[kRegEvents];
     const uint64_t ovf = uint64_t(rg[kRegOverflowLo]) | (uint64_t(rg[kRegOverflowHi]) << 32);
     const size_t evBase = size_t(region) * kPtBlock * sb.ev_per_path;
-    const bool stage = Mode == kUnwindExact && sb.stage != 0u;
     PathSums sum;
     // block-uniform loop (one wave per block): 64 events per round, then each lane adds its own
     // path's contributions in slot order, which is the order the megakernel adds them in
@@ -728,14 +864,13 @@ solve_unwind_kernel(PtScene sc, PtFrame fr, SolveBuffers sb) {
             const size_t e = evBase + k;
             const uint32_t meta = ev_get(sb, e, kEvMeta);
             who = meta & 63u;
-            if (((ovf >> who) & 1u) || ((meta >> 13) & 3u) == kEvKindVoid || (stage && is_walk_event(meta))) {
-                who = kPtBlock;  // left to the megakernel, void, or the walk-unwind kernel's
+            if (((ovf >> who) & 1u) || ((meta >> 13) & 3u) == kEvKindVoid) {
+                who = kPtBlock;  // left to the megakernel, or void
             } else {
                 unwind_event<N, Mode>(sc, fr, sb, e, meta, region, c);
-                if (stage) contrib_put(sb, e, c);
             }
         }
-        if (Mode == kUnwindQuery || stage) continue;
+        if (Mode == kUnwindQuery) continue;
         owner[lane] = who;
         part[0][lane] = c[0];
         part[1][lane] = c[1];
@@ -744,29 +879,9 @@ solve_unwind_kernel(PtScene sc, PtFrame fr, SolveBuffers sb) {
         sum.add_round(owner, part, min(count - base, uint32_t(kPtBlock)), lane);
         __syncthreads();
     }
-    if (Mode == kUnwindQuery || stage) return;
+    if (Mode == kUnwindQuery) return;
     const uint32_t li = region * kPtBlock + lane;
     if (li < fr.n_paths && !((ovf >> lane) & 1u)) fr.color[path_pixel(fr.width, fr.height, fr.path_base + li)] = make_float4(sum.r, sum.g, sum.b, 1.f);
-}
-
-// Staged unwind, after the walk kernel: the contributions of the walks that succeeded, one lane per
-// queued walk (the void ones add nothing).
-template <int N>
-__global__ void __launch_bounds__(kPtBlock) __attribute__((amdgpu_waves_per_eu(2, 2)))
-solve_walk_unwind_kernel(PtScene sc, PtFrame fr, SolveBuffers sb) {
-    const uint32_t total = sb.walk.counters[0];
-    const size_t regionEvents = size_t(kPtBlock) * sb.ev_per_path;
-    for (uint32_t k = blockIdx.x * kPtBlock + threadIdx.x; k < total; k += gridDim.x * kPtBlock) {
-        const size_t e = sb.walk.items[k];
-        const uint32_t meta = ev_get(sb, e, kEvMeta);
-        if (((meta >> 13) & 3u) == kEvKindVoid) continue;
-        const uint32_t region = uint32_t(e / regionEvents), who = meta & 63u;
-        const uint32_t* rg = sb.region + size_t(region) * kRegWords;
-        if ((rg[who < 32u ? kRegOverflowLo : kRegOverflowHi] >> (who & 31u)) & 1u) continue;  // the megakernel's
-        float c[3] = {0.f, 0.f, 0.f};
-        unwind_event<N, kUnwindExact>(sc, fr, sb, e, meta, region, c);
-        contrib_put(sb, e, c);
-    }
 }
 
 // Staged unwind, last: each path's contributions summed in slot order, the colour written.

@@ -358,13 +358,31 @@ __device__ bool targets_of(const float* __restrict__ Mrow, double* y) {
     return ok;
 }
 
+// The column sums of a block's rows, each as sixteen sums of every sixteenth row added in order.
+__device__ void column_sums(double (&ys)[kEw][kOut], int rows, double* __restrict__ out) {
+    __shared__ double part[kEw / kOut][kOut];
+    const int c = threadIdx.x % kOut, q = threadIdx.x / kOut;
+    double acc = 0.0;
+    for (int r = q; r < rows; r += kEw / kOut) acc += ys[r][c];
+    part[q][c] = acc;
+    __syncthreads();
+    if (threadIdx.x < kOut) {
+        double sum = 0.0;
+        for (int k = 0; k < kEw / kOut; ++k) sum += part[k][threadIdx.x];
+        out[threadIdx.x] = sum;
+    }
+}
+
 // Pass 1, per block of kEw rows: valid count, column sums of the targets (double), and the box of
-// the valid rows' inputs. Sums run over the block's rows in order (deterministic).
+// the valid rows' inputs, in a fixed order. Every thread takes a sixteenth of a column and an eighth of a
+// feature (one thread per column and feature walked the block's 256 rows one after the other, with a
+// dependent load each: 264,000 rows 152 us).
 __global__ void __launch_bounds__(kEw) prep_sums_kernel(int n, const float* __restrict__ X, const float* __restrict__ M,
                                                         double* __restrict__ psum, float* __restrict__ plo, float* __restrict__ phi,
                                                         uint32_t* __restrict__ pcount) {
     __shared__ double ys[kEw][kOut];
     __shared__ uint8_t valid[kEw];
+    __shared__ float lo_s[kEw / 32][32], hi_s[kEw / 32][32];
     const int t = threadIdx.x, i = blockIdx.x * kEw + t;
     double y[kOut];
     bool ok = false;
@@ -374,25 +392,33 @@ __global__ void __launch_bounds__(kEw) prep_sums_kernel(int n, const float* __re
     valid[t] = ok ? 1 : 0;
     __syncthreads();
     const int rows = min(kEw, n - int(blockIdx.x) * kEw);
-    if (t < kOut) {
-        double acc = 0.0;
-        for (int r = 0; r < rows; ++r) acc += ys[r][t];
-        psum[size_t(blockIdx.x) * kOut + t] = acc;
-    } else if (t >= 32 && t < 32 + kIn) {
-        const int f = t - 32;
+    column_sums(ys, rows, psum + size_t(blockIdx.x) * kOut);
+    // the box: feature t % 32 (< 22) over rows t / 32 + 8 k, then the eight partial boxes
+    {
+        const int f = t & 31, q = t >> 5;
         float lo = __builtin_inff(), hi = -__builtin_inff();
-        for (int r = 0; r < rows; ++r)
-            if (valid[r]) {
-                const float v = X[(size_t(blockIdx.x) * kEw + r) * kIn + f];
-                lo = fminf(lo, v);
-                hi = fmaxf(hi, v);
-            }
-        plo[size_t(blockIdx.x) * kIn + f] = lo;
-        phi[size_t(blockIdx.x) * kIn + f] = hi;
+        if (f < kIn)
+            for (int r = q; r < rows; r += kEw / 32)
+                if (valid[r]) {
+                    const float v = X[(size_t(blockIdx.x) * kEw + r) * kIn + f];
+                    lo = fminf(lo, v);
+                    hi = fmaxf(hi, v);
+                }
+        lo_s[q][f] = lo;
+        hi_s[q][f] = hi;
+    }
+    const int c = __syncthreads_count(valid[t] != 0);
+    if (t < kIn) {
+        float lo = lo_s[0][t], hi = hi_s[0][t];
+#pragma unroll
+        for (int q = 1; q < kEw / 32; ++q) {
+            lo = fminf(lo, lo_s[q][t]);
+            hi = fmaxf(hi, hi_s[q][t]);
+        }
+        plo[size_t(blockIdx.x) * kIn + t] = lo;
+        phi[size_t(blockIdx.x) * kIn + t] = hi;
     } else if (t == 64) {
-        uint32_t c = 0;
-        for (int r = 0; r < rows; ++r) c += valid[r];
-        pcount[blockIdx.x] = c;
+        pcount[blockIdx.x] = uint32_t(c);
     }
 }
 
@@ -498,12 +524,7 @@ __global__ void __launch_bounds__(kEw) prep_dev_kernel(int n, const float* __res
         for (int w = 0; w < wave; ++w) before += wcount[w];
         idx[boffset[blockIdx.x] + before] = uint32_t(i);
     }
-    const int rows = min(kEw, n - int(blockIdx.x) * kEw);
-    if (t < kOut) {
-        double acc = 0.0;
-        for (int r = 0; r < rows; ++r) acc += ys[r][t];
-        psum[size_t(blockIdx.x) * kOut + t] = acc;
-    }
+    column_sums(ys, min(kEw, n - int(blockIdx.x) * kEw), psum + size_t(blockIdx.x) * kOut);
 }
 
 // One block of 1024 threads: the standard deviations (population), scaled by the output weights,
@@ -596,11 +617,14 @@ __global__ void shuffle_kernel(uint32_t n, int half, uint32_t key, uint32_t* __r
 // consecutive samples of one feature). A hidden unit's ReLU mask is one bit in the lane that
 // computed it, which is the lane that computes its gradient.
 //
-// It is bound by the chain of ten barriers per tile with one group per CU (125 KB of LDS): a batch of
-// 16,384 is 256 tiles over 128 groups. Before, a step was eighteen dependent launches (a GEMM per
-// product and gradient, 9 us each, every activation through memory in two layouts): 141 us.
+// It is bound by the chain of ten barriers per tile, about 2 us each, with one group per CU (125 KB of
+// LDS) and one wave per SIMD. A batch of 16,384 rows is one tile for each of 256 groups: 30 us and 9 us
+// for the reduction, with 128 groups 43 and 6 us. Loading the next product's weights a phase ahead,
+// across barriers that order LDS only, spilled registers and took 46 us. Before, a step was eighteen
+// dependent launches (a GEMM per product and gradient, 9 us each, every activation through memory in
+// two layouts): 141 us.
 // ---------------------------------------------------------------------------------------
-constexpr int kGroupsMax = 128;  // partials to sum: more groups write and read more of them (20 MB at 128)
+constexpr int kGroupsMax = 256;  // partials to sum (40 MB at 256): one group per CU
 constexpr int kTRow = kFTile + 8;  // feature-major LDS rows
 
 // The layout of one group's partial: W4, W3, W2, W1 (its 32 padded inputs), then the biases b4, b3, b2, b1.

@@ -460,3 +460,47 @@ def test_lambda_pdf_limits():
         assert lp[0] > 0 and np.all(lp == lp[0]), (mat.type, lp)
         _, _, lp2 = O.material_eval(bytes(mat), prof, 2, wi, wo, 0x02, lam, S, 30.0)
         assert len(set(lp2.tolist())) > 1, (mat.type, lp2)  # the scattering pdf depends on the wavenumber
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 63, 64, 255, 256, 257, 1000])
+def test_gpu_material_batches_do_not_depend_on_the_order_of_queries(gpu, n):
+    """The batch kernels sort each block's 256 queries by material: every query gets its own result
+    whatever stands beside it -- a batch and its reverse agree bit for bit, a sample batch agrees with the
+    first part of a longer one (a query's random numbers come from its index) -- and a material index
+    out of range still gives zeros."""
+    import torch
+    from pltfalcor_amd import _lib
+    from pltfalcor_amd import materials as M
+    from pltfalcor_amd.bsdf import MaterialTable, default_context
+    mats = _all_materials()
+    table = MaterialTable(default_context(), M.pack(mats))
+    rng = np.random.default_rng(n)
+
+    def fill(planes, count):
+        q = rng.uniform(0.1, 1.0, (planes, count)).astype(np.float32)
+        v = rng.normal(size=(3, count))
+        q[0:3] = v / np.linalg.norm(v, axis=0)
+        return q
+
+    q = fill(_lib.MQ_PLANES, n)
+    v = rng.normal(size=(3, n))
+    q[3:6] = v / np.linalg.norm(v, axis=0)
+    b = q.view(np.uint32)
+    b[_lib.MQ_LOBE] = rng.choice([0x01, 0x02, 0x04, 0x33, 0x40], n)
+    b[_lib.MQ_MAT] = rng.integers(0, len(mats) + 1, n)  # one past the table among them
+    q[_lib.MQ_LAMBDA:_lib.MQ_LAMBDA + 4] = rng.uniform(380, 720, (4, n))
+    q[_lib.MQ_AREA] = rng.uniform(1, 100, n)
+    a = table.eval(torch.from_numpy(q).cuda()).cpu().numpy()
+    r = table.eval(torch.from_numpy(q[:, ::-1].copy()).cuda()).cpu().numpy()[:, ::-1]
+    assert np.array_equal(a.view(np.uint32), np.ascontiguousarray(r).view(np.uint32))
+    assert np.all(a[:, b[_lib.MQ_MAT] == len(mats)] == 0)
+    m = n + 300
+    q = fill(_lib.MSQ_PLANES, m)
+    b = q.view(np.uint32)
+    b[_lib.MSQ_MAT] = rng.integers(0, len(mats) + 1, m)
+    q[_lib.MSQ_LAMBDA] = rng.uniform(380, 720, m)
+    long = table.sample(torch.from_numpy(q).cuda(), frame=3).cpu().numpy()
+    short = table.sample(torch.from_numpy(q[:, :n].copy()).cuda(), frame=3).cpu().numpy()
+    assert np.array_equal(long[:, :n].copy().view(np.uint32), short.view(np.uint32))
+    assert np.all(long.view(np.uint32)[-1, b[_lib.MSQ_MAT] == len(mats)] == 0)

@@ -733,7 +733,7 @@ def main():
     else:
         kb["megakernel"] = SOLVE_BYTES_PER_SEGMENT * seg_per_exec + SOLVE_BYTES_PER_PIXEL * pixels
     knames = {"sample": "sample_kernel", "light": "solve_sample_kernel<4, false>",
-              "walk": "solve_walk_kernel (the non-walk events' solve_unwind_kernel<4> runs beside it on a second "
+              "walk": "solve_walk_kernel (the non-walk events' solve_unwind_staged_kernel<4> runs beside it on a second "
                       "stream)",
               "unwind": "solve_walk_unwind_kernel<4>, the join with the second stream, solve_sum_kernel",
               "megakernel": "solve_kernel<4, false>" + (" (fallback of the split pass)" if split and not launch["graph"] else "")}

@@ -3,7 +3,7 @@
 //
 // Every MFMA operand is bf16 and contiguous along the contracted dimension, so that a fragment (8
 // consecutive k of one row) is one 16 B load. Accumulation is FP32 (v_mfma_f32_16x16x32_bf16); master
-// weights and Adam moments are FP32; weight gradients are partial sums per workgroup reduced in a
+// weights and Adam moments are FP32; weight gradients are split sums over the batch reduced in a
 // fixed order (the result does not depend on scheduling).
 //
 // Layers (parameter order of plt_surrogate_params): W1 [128 x 22], b1 [128], W2 [128 x 128], b2,
@@ -287,7 +287,7 @@ __global__ void __launch_bounds__(kFThreads) mlp_infer_kernel(int n, const float
 // ---------------------------------------------------------------------------------------
 constexpr int kEw = 256;
 
-// bf16 operand copies of one layer: W [out x in_pad] and Wt [in x out_pad] from the master
+// bf16 operand copies of one layer: W [out x in_pad] and, if Wt, Wt [in x out_pad] from the master
 // weights [out x in] (padding zero).
 __global__ void cast_weights_kernel(int out, int in, int in_pad, int out_pad, const float* __restrict__ Wm, __bf16* __restrict__ W,
                                     __bf16* __restrict__ Wt) {
@@ -296,7 +296,7 @@ __global__ void cast_weights_kernel(int out, int in, int in_pad, int out_pad, co
     const int o = e / in_pad, i = e % in_pad;
     const __bf16 v = static_cast<__bf16>(o < out && i < in ? Wm[size_t(o) * in + i] : 0.f);
     if (o < out) W[size_t(o) * in_pad + i] = v;
-    if (i < in) Wt[size_t(i) * out_pad + o] = v;
+    if (Wt && i < in) Wt[size_t(i) * out_pad + o] = v;
 }
 
 }  // namespace mlp
@@ -326,7 +326,7 @@ int dev_alloc(plt_surrogate* s, T** p, size_t count) {
 
 int cast_all(plt_surrogate* s, hipStream_t st) {
     struct L { size_t off; int out, in, in_pad, out_pad; __bf16 *W, *Wt; };
-    const L layers[4] = {{kOffW1, kHid, kIn, kInPad, kHid, s->W1, s->W1t},
+    const L layers[4] = {{kOffW1, kHid, kIn, kInPad, kHid, s->W1, nullptr},
                          {kOffW2, kHid, kHid, kHid, kHid, s->W2, s->W2t},
                          {kOffW3, kHid, kHid, kHid, kHid, s->W3, s->W3t},
                          {kOffW4, kOut, kHid, kHid, kOutPad, s->W4, s->W4t}};
@@ -358,25 +358,24 @@ __device__ bool targets_of(const float* __restrict__ Mrow, double* y) {
     return ok;
 }
 
-// The column sums of a block's rows, each as sixteen sums of every sixteenth row added in order.
-__device__ void column_sums(double (&ys)[kEw][kOut], int rows, double* __restrict__ out) {
-    __shared__ double part[kEw / kOut][kOut];
-    const int c = threadIdx.x % kOut, q = threadIdx.x / kOut;
+// The column sums of a block's rows, in row order; sixteen rows are read before their adds (an FP64 add
+// per row is the chain, about a microsecond a block).
+__device__ void column_sums(const double (&ys)[kEw][kOut], int rows, double* __restrict__ out) {
+    if (threadIdx.x >= kOut) return;
     double acc = 0.0;
-    for (int r = q; r < rows; r += kEw / kOut) acc += ys[r][c];
-    part[q][c] = acc;
-    __syncthreads();
-    if (threadIdx.x < kOut) {
-        double sum = 0.0;
-        for (int k = 0; k < kEw / kOut; ++k) sum += part[k][threadIdx.x];
-        out[threadIdx.x] = sum;
+    for (int r0 = 0; r0 < rows; r0 += 16) {
+        double v[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) v[j] = ys[r0 + j][threadIdx.x];  // kEw rows are there
+#pragma unroll
+        for (int j = 0; j < 16; ++j) acc = r0 + j < rows ? acc + v[j] : acc;
     }
+    out[threadIdx.x] = acc;
 }
 
 // Pass 1, per block of kEw rows: valid count, column sums of the targets (double), and the box of
-// the valid rows' inputs, in a fixed order. Every thread takes a sixteenth of a column and an eighth of a
-// feature (one thread per column and feature walked the block's 256 rows one after the other, with a
-// dependent load each: 264,000 rows 152 us).
+// the valid rows' inputs. Every thread takes an eighth of a feature's box (one thread per feature walked
+// the block's 256 rows one after the other, with a dependent load each: 264,000 rows 152 us).
 __global__ void __launch_bounds__(kEw) prep_sums_kernel(int n, const float* __restrict__ X, const float* __restrict__ M,
                                                         double* __restrict__ psum, float* __restrict__ plo, float* __restrict__ phi,
                                                         uint32_t* __restrict__ pcount) {
@@ -603,39 +602,54 @@ __global__ void shuffle_kernel(uint32_t n, int half, uint32_t key, uint32_t* __r
 }
 
 // ---------------------------------------------------------------------------------------
-// Fused training step: forward pass, loss, backward pass and the weight gradients of one batch in
-// one kernel. A workgroup of four waves takes every gridDim.x-th tile of 64 samples; a tile's
-// activations never leave LDS, and the gradients of all 38,032 parameters are summed over the
-// group's tiles in its waves' accumulators (176 registers a lane) and written once, as one partial
-// per group. grad_reduce_kernel sums the partials in group order (and, in training, applies Adam), so
-// a step is two launches.
+// Training step: three launches. mlp_train_kernel runs the forward pass, the loss and the backward
+// pass, a workgroup of four waves per tile of 64 samples, whose activations and back-propagated
+// gradients go from layer to layer in LDS and to memory once; mlp_weight_grad_kernel contracts them
+// over the batch into split sums of the weights' gradients; grad_reduce_kernel adds the splits in
+// order (and, in training, applies Adam).
 //
 // Products are computed transposed as in mlp_infer_kernel (weights the A operand, out[feature x
 // sample]); wave w holds features 32w..32w+31. Each activation and each back-propagated gradient is
 // stored twice: sample-major rows (the next product's B operand: 8 consecutive features) and
 // feature-major rows (the weight gradients contract over samples, so both their operands are 8
-// consecutive samples of one feature). A hidden unit's ReLU mask is one bit in the lane that
-// computed it, which is the lane that computes its gradient.
+// consecutive samples of one feature), which are also what goes to memory. A hidden unit's ReLU mask
+// is one bit in the lane that computed it, which is the lane that computes its gradient.
 //
-// It is bound by the chain of ten barriers per tile, about 2 us each, with one group per CU (125 KB of
-// LDS) and one wave per SIMD. A batch of 16,384 rows is one tile for each of 256 groups: 30 us and 9 us
-// for the reduction, with 128 groups 43 and 6 us. Loading the next product's weights a phase ahead,
-// across barriers that order LDS only, spilled registers and took 46 us. Before, a step was eighteen
-// dependent launches (a GEMM per product and gradient, 9 us each, every activation through memory in
-// two layouts): 141 us.
+// Every sum has an order that does not depend on the grid: a product adds its blocks of 32 k in order
+// and its bias last, a split is a chain over at most 1/64 of the batch (rounded up to 32 rows), and the
+// splits, the tiles' bias sums and the losses are added as grad_reduce_kernel says. Groups that kept their
+// tiles' weight gradients in accumulators (two launches, 30 and 9 us for 16,384 rows) rounded otherwise for
+// another number of groups, and summed their losses in one FP32 chain.
+//
+// A batch of 16,384 rows: 19.9, 7.4 and 5.9 us. The first is bound by the chain of its nine LDS barriers
+// (256 tiles, one per CU; 14 us for a single tile), so a product's weights are loaded a phase ahead, and the
+// barriers leave the stores of what is kept in flight. The second reads 26 MB and writes 10, 3.3 TB/s
+// after the latency of its two rounds of loads. (Eighteen launches, a GEMM per product and gradient with
+// every activation through memory in two layouts: 141 us.)
 // ---------------------------------------------------------------------------------------
-constexpr int kGroupsMax = 256;  // partials to sum (40 MB at 256): one group per CU
 constexpr int kTRow = kFTile + 8;  // feature-major LDS rows
 
-// The layout of one group's partial: W4, W3, W2, W1 (its 32 padded inputs), then the biases b4, b3, b2, b1.
+// What a tile leaves in memory for the weight gradients: its 64 samples of every feature, as the MFMA
+// fragments that contract over samples, each 1 KB in lane order: [16 features][32 samples][lane][8 samples].
+constexpr int kActX = 0, kActH1 = kActX + kInPad * kFTile, kActH2 = kActH1 + kHid * kFTile, kActH3 = kActH2 + kHid * kFTile,
+              kActDY = kActH3 + kHid * kFTile, kActG3 = kActDY + kOut * kFTile, kActG2 = kActG3 + kHid * kFTile,
+              kActG1 = kActG2 + kHid * kFTile, kActTile = kActG1 + kHid * kFTile;  // 104,448 B
+
+// One split's weight gradients: W4, W3, W2, W1 (its 32 padded inputs). The biases' sums, a row per tile
+// (b4, b3, b2, b1), follow them in grad_reduce_kernel's list of elements.
 constexpr int kPartW4 = 0, kPartW3 = kPartW4 + kOut * kHid, kPartW2 = kPartW3 + kHid * kHid, kPartW1 = kPartW2 + kHid * kHid,
               kGradTotal = kPartW1 + kHid * kInPad;  // 38,912
 constexpr int kBiasCols = kOut + 3 * kHid;
-constexpr int kPartTotal = kGradTotal + kBiasCols;
+constexpr int kSplitTarget = 64;  // splits of the batch at most
+// Rows of one split (a multiple of 32).
+int split_len(uint32_t n) { return int((n / kKStep + kSplitTarget - 1) / kSplitTarget * kKStep); }
+int tiles_of(uint32_t n) { return int((n + kFTile - 1) / kFTile); }
+constexpr int kLossRows = 256;  // rows whose losses are summed in FP32; those sums are added in double
+int loss_blocks(uint32_t n) { return int((n + kLossRows - 1) / kLossRows); }
 
 // Device-side state of plt_surrogate_train: every launch of a training step reads what it needs
 // from here, so one captured step replays as every step. The train kernel reads `step` and publishes
-// the step it runs, its learning rate and Adam's corrections (group 0); the reduction reads those and
+// the step it runs, its learning rate and Adam's corrections (tile 0); the reduction reads those and
 // advances `step`.
 struct TrainState {
     uint32_t step, steps_per_epoch, steps_total, batch, n_valid, seed, adam_t0;
@@ -643,87 +657,82 @@ struct TrainState {
     uint32_t now;
     float lr, c1, c2;
 };
+static_assert(sizeof(TrainState) <= kTrainStateWords * 4, "train state size");
 
 struct TrainArgs {
     int n;                 // rows of the batch
-    const float *X, *T;    // inputs [. x 22] and targets [. x 16]
+    const float *X, *T;    // inputs [. x 22] and targets [. x 16], at any address that floats may have
     const uint32_t* idx;   // with st: row i of the batch is idx[shuffle(step's i-th position)]
     int half;
     TrainState* st;
     const __bf16 *W1, *W2, *W3, *W4, *W2t, *W3t, *W4t;
     const float *b1, *b2, *b3, *b4;
-    float* part;           // [gridDim.x x kPartTotal]
-    float* loss_part;      // [gridDim.x]
+    __bf16* act;           // [tiles x kActTile]
+    float* bias_part;      // [tiles x kBiasCols]
+    float* row_loss;       // [n]
 };
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
-__global__ void __launch_bounds__(kFThreads, 1) mlp_train_kernel(TrainArgs g) {
-    __shared__ __bf16 xs[kFTile * kXRow], xt[kInPad * kTRow];
+// A barrier that orders the workgroup's LDS accesses only: loads from and stores to memory stay in
+// flight across it. (Within mlp_train_kernel no thread reads what another wrote to memory.)
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+__global__ void __launch_bounds__(kFThreads, 2) mlp_train_kernel(TrainArgs g) {
+    __shared__ __bf16 xs[kFTile * kXRow];                              // the inputs; after the first layer dY, K padded to 32
     __shared__ __bf16 sa[kFTile * kHRow], sb[kFTile * kHRow];          // sample-major, ping-pong
-    __shared__ __bf16 h1t[kHid * kTRow], h2t[kHid * kTRow], h3t[kHid * kTRow], gt[kHid * kTRow];
-    __shared__ __bf16 dy[kFTile * kXRow], dyt[kOut * kTRow];
+    __shared__ __bf16 f0[kHid * kTRow], f1[kHid * kTRow];              // feature-major, ping-pong
+    __shared__ __bf16 dyt[kOut * kTRow];
     __shared__ uint32_t rows[kFTile];
-    __shared__ float red[kFThreads / 64][1 + kOut];
     const int t = threadIdx.x, w = t >> 6, lane = t & 63;
     const int fr = lane & 15, fg = lane >> 4, fk = 8 * fg;
-    uint32_t step = 0, epoch_pos = 0, key = 0, n_valid = 0;
-    if (g.st) {
+    const int r0 = int(blockIdx.x) * kFTile;
+    __bf16* act = g.act + size_t(blockIdx.x) * kActTile;
+    float* bias_part = g.bias_part + size_t(blockIdx.x) * kBiasCols;
+    // rows past n repeat the last one; what they give is zeroed
+    if (t < kFTile) {
+        uint32_t row = uint32_t(min(r0 + t, g.n - 1));
+        if (g.st) {
+            const TrainState s = *g.st;
+            row = g.idx[shuffle_index((s.step % s.steps_per_epoch) * s.batch + row, s.n_valid, g.half, epoch_key(s.seed, s.step / s.steps_per_epoch))];
+        }
+        rows[t] = row;
+    } else if (t == kFTile && blockIdx.x == 0 && g.st) {
+        // the cosine-decayed rate (at least 1e-6) and the corrections of Adam step adam_t0 + step + 1
         const TrainState s = *g.st;
-        step = s.step;
-        n_valid = s.n_valid;
-        epoch_pos = (step % s.steps_per_epoch) * s.batch;
-        key = epoch_key(s.seed, step / s.steps_per_epoch);
-        if (blockIdx.x == 0 && t == 0) {
-            // the cosine-decayed rate (at least 1e-6) and the corrections of Adam step adam_t0 + step + 1
-            const double tt = double(s.adam_t0) + double(step) + 1.0;
-            g.st->now = step;
-            g.st->c1 = float(1.0 - pow(double(0.9f), tt));
-            g.st->c2 = float(1.0 - pow(double(0.999f), tt));
-            const double cs = cos(3.14159265358979323846 * double(step) / double(max(1u, s.steps_total)));
-            g.st->lr = float(fmax(double(s.lr0) * 0.5 * (1.0 + cs), 1e-6));
-        }
+        const double tt = double(s.adam_t0) + double(s.step) + 1.0;
+        g.st->now = s.step;
+        g.st->c1 = float(1.0 - pow(double(0.9f), tt));
+        g.st->c2 = float(1.0 - pow(double(0.999f), tt));
+        const double cs = cos(3.14159265358979323846 * double(s.step) / double(max(1u, s.steps_total)));
+        g.st->lr = float(fmax(double(s.lr0) * 0.5 * (1.0 + cs), 1e-6));
     }
-    // outputs 16..31 of dY pad its K dimension with zeros
-    for (int i = t; i < kFTile * kXRow; i += kFThreads) dy[i] = static_cast<__bf16>(0.f);
-    f32x4 c1[2], c2[2], c3[2], c4;
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int f = 32 * w + 16 * cb + 4 * fg + r;
-            c1[cb][r] = g.b1[f];
-            c2[cb][r] = g.b2[f];
-            c3[cb][r] = g.b3[f];
-        }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) c4[r] = g.b4[4 * fg + r];
+    using K1 = std::integral_constant<int, 1>;
+    using K4 = std::integral_constant<int, 4>;
     const f32x4 zero{0.f, 0.f, 0.f, 0.f};
-    f32x4 dw1[2][2], dw2[2][8], dw3[2][8], dw4[2], db1[2], db2[2], db3[2], db4 = zero;
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-#pragma unroll
-        for (int b = 0; b < 8; ++b) dw2[a][b] = dw3[a][b] = zero;
-        dw1[a][0] = dw1[a][1] = dw4[a] = db1[a] = db2[a] = db3[a] = zero;
-    }
-    float loss = 0.f;
-    const float scale = 2.f / (float(g.n) * float(kOut));
-
-    // out[32w..32w+31 x 64 samples] from kb blocks of 32 sample-major inputs and the weight rows Wm
-    auto product = [&](auto kblocks, const __bf16* in, int in_row, const __bf16* Wm, int ldw, const f32x4* init, f32x4 (&acc)[2][4]) {
-        constexpr int kK = decltype(kblocks)::value;
-        bf16x8 wf[2][kK];
+    // a product's weight fragments, rows 32w..32w+31 of Wm: loaded a phase ahead
+    bf16x8 wf[2][4];
+    auto weights = [&](auto kblocks, const __bf16* Wm, int ldw) {
 #pragma unroll
         for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
-            for (int kb = 0; kb < kK; ++kb)
+            for (int kb = 0; kb < decltype(kblocks)::value; ++kb)
                 wf[cb][kb] = *reinterpret_cast<const bf16x8*>(Wm + size_t(32 * w + 16 * cb + fr) * ldw + 32 * kb + fk);
+    };
+    // out[32w..32w+31 x 64 samples] from blocks of 32 sample-major inputs and the fragments
+    auto product = [&](auto kblocks, const __bf16* in, int in_row, f32x4 (&acc)[2][4]) {
 #pragma unroll
         for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
-            for (int s = 0; s < 4; ++s) acc[cb][s] = init ? init[cb] : zero;
+            for (int s = 0; s < 4; ++s) acc[cb][s] = zero;
 #pragma unroll
         for (int s = 0; s < 4; ++s)
 #pragma unroll
-            for (int kb = 0; kb < kK; ++kb) {
+            for (int kb = 0; kb < decltype(kblocks)::value; ++kb) {
                 const bf16x8 b = *reinterpret_cast<const bf16x8*>(in + (16 * s + fr) * in_row + 32 * kb + fk);
 #pragma unroll
                 for (int cb = 0; cb < 2; ++cb) acc[cb][s] = mfma(wf[cb][kb], b, acc[cb][s]);
@@ -736,9 +745,7 @@ __global__ void __launch_bounds__(kFThreads, 1) mlp_train_kernel(TrainArgs g) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) fm[(f + r) * kTRow + row] = h[r];
     };
-    auto forward = [&](auto kblocks, const __bf16* in, int in_row, const __bf16* Wm, int ldw, const f32x4* bias, __bf16* sm, __bf16* fm) {
-        f32x4 acc[2][4];
-        product(kblocks, in, in_row, Wm, ldw, bias, acc);
+    auto relu = [&](const f32x4 (&acc)[2][4], const float* bias, __bf16* sm, __bf16* fm) {
         uint32_t mask = 0;
 #pragma unroll
         for (int cb = 0; cb < 2; ++cb)
@@ -747,191 +754,253 @@ __global__ void __launch_bounds__(kFThreads, 1) mlp_train_kernel(TrainArgs g) {
                 bf16x4 h;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    h[r] = static_cast<__bf16>(relu_bits(acc[cb][s][r]));
+                    const float v = acc[cb][s][r] + bias[32 * w + 16 * cb + 4 * fg + r];
+                    h[r] = static_cast<__bf16>(fmaxf(v, 0.f));
                     mask |= static_cast<float>(h[r]) > 0.f ? 1u << (16 * cb + 4 * s + r) : 0u;
                 }
                 store(h, cb, s, sm, fm);
             }
         return mask;
     };
-    auto backward = [&](auto kblocks, const __bf16* in, int in_row, const __bf16* Wt, int ldw, uint32_t mask, __bf16* sm, __bf16* fm, f32x4 (&db)[2]) {
-        f32x4 acc[2][4];
-        product(kblocks, in, in_row, Wt, ldw, nullptr, acc);
+    auto masked = [&](const f32x4 (&acc)[2][4], uint32_t mask, __bf16* sm, __bf16* fm) {
 #pragma unroll
         for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
                 bf16x4 h;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    h[r] = static_cast<__bf16>((mask >> (16 * cb + 4 * s + r)) & 1u ? acc[cb][s][r] : 0.f);
-                    db[cb][r] += static_cast<float>(h[r]);
-                }
+                for (int r = 0; r < 4; ++r) h[r] = static_cast<__bf16>((mask >> (16 * cb + 4 * s + r)) & 1u ? acc[cb][s][r] : 0.f);
                 store(h, cb, s, sm, fm);
             }
     };
-    // dW[32w..32w+31 x 16 B..] += G H^T over the tile's 64 samples (feature-major operands)
-    auto weight_grad = [&](auto nb, const __bf16* gm, const __bf16* hm, auto& dw) {
-        constexpr int kB = decltype(nb)::value;
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-            bf16x8 a[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) a[i] = *reinterpret_cast<const bf16x8*>(gm + (32 * w + 16 * i + fr) * kTRow + 32 * kb + fk);
-#pragma unroll
-            for (int b = 0; b < kB; ++b) {
-                const bf16x8 h = *reinterpret_cast<const bf16x8*>(hm + (16 * b + fr) * kTRow + 32 * kb + fk);
-#pragma unroll
-                for (int i = 0; i < 2; ++i) dw[i][b] = mfma(a[i], h, dw[i][b]);
-            }
-        }
+    // `count` feature-major rows to memory as fragments, 16 B per thread and round
+    auto keep = [&](const __bf16* fm, int count, __bf16* dst) {
+        for (int c = t; c < count * (kFTile / 8); c += kFThreads)
+            *reinterpret_cast<bf16x8*>(dst + 8 * c) =
+                *reinterpret_cast<const bf16x8*>(fm + (16 * (c >> 7) + fr) * kTRow + 32 * ((c >> 6) & 1) + fk);
     };
-    using K1 = std::integral_constant<int, 1>;
-    using K2 = std::integral_constant<int, 2>;
-    using K4 = std::integral_constant<int, 4>;
-    using K8 = std::integral_constant<int, 8>;
+    // a bias gradient's sums over the tile: thread t adds half t % 2 of feature t / 2, as the four sums of
+    // rows 4 q .. 4 q + 3 and 16 + 4 q .. of the half, those in pairs, then the halves
+    auto bias_sums = [&](const __bf16* fm, float* dst) {
+        const __bf16* row = fm + (t >> 1) * kTRow + 32 * (t & 1);
+        float s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const bf16x8 v = *reinterpret_cast<const bf16x8*>(row + 8 * c);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) s[(2 * c + j / 4) & 3] += static_cast<float>(v[j]);
+        }
+        const float h = (s[0] + s[1]) + (s[2] + s[3]);
+        const float both = h + __shfl_xor(h, 1);
+        if ((t & 1) == 0) dst[t >> 1] = both;
+    };
+    f32x4 acc[2][4];
+    weights(K1{}, g.W1, kInPad);
+    lds_barrier();
+    {
+        // thread t stages input features 2p, 2p + 1 (p = t % 16) of rows t / 16 + 16 j; rows past n
+        // and padding features are zero
+        const int p = t & 15, sr = t >> 4;
+        const bool in = 2 * p < kIn;
+        f32x2u v[kFTile / 16];
+#pragma unroll
+        for (int j = 0; j < kFTile / 16; ++j)
+            v[j] = *reinterpret_cast<const f32x2u*>(g.X + size_t(rows[sr + 16 * j]) * kIn + (in ? 2 * p : 0));
+#pragma unroll
+        for (int j = 0; j < kFTile / 16; ++j) {
+            const int r = sr + 16 * j;
+            const bool live = in && r0 + r < g.n;
+            bf16x2 pv;
+            pv[0] = static_cast<__bf16>(live ? v[j].x : 0.f);
+            pv[1] = static_cast<__bf16>(live ? v[j].y : 0.f);
+            *reinterpret_cast<bf16x2*>(xs + r * kXRow + 2 * p) = pv;
+            f1[(2 * p) * kTRow + r] = pv[0];
+            f1[(2 * p + 1) * kTRow + r] = pv[1];
+        }
+    }
+    // the lane's four targets: outputs 4 fg.. of sample 16 w + fr
+    const int srow = 16 * w + fr;
+    const f32x4u target = *reinterpret_cast<const f32x4u*>(g.T + size_t(rows[srow]) * kOut + 4 * fg);
+    lds_barrier();
+    product(K1{}, xs, kXRow, acc);
+    weights(K4{}, g.W2, kHid);
+    const uint32_t m1 = relu(acc, g.b1, sa, f0);
+    keep(f1, kInPad, act + kActX);
+    lds_barrier();
+    product(K4{}, sa, kHRow, acc);
+    weights(K4{}, g.W3, kHid);
+    const uint32_t m2 = relu(acc, g.b2, sb, f1);
+    keep(f0, kHid, act + kActH1);
+    lds_barrier();
+    product(K4{}, sb, kHRow, acc);
+    bf16x8 w4[4];
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) w4[kb] = *reinterpret_cast<const bf16x8*>(g.W4 + size_t(fr) * kHid + 32 * kb + fk);
+    const uint32_t m3 = relu(acc, g.b3, sa, f0);
+    keep(f1, kHid, act + kActH2);
+    lds_barrier();
+    {
+        f32x4 y = zero;
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) y = mfma(w4[kb], *reinterpret_cast<const bf16x8*>(sa + srow * kHRow + 32 * kb + fk), y);
+        weights(K1{}, g.W4t, kOutPad);
+        const bool live = r0 + srow < g.n;
+        const float scale = 2.f / (float(g.n) * float(kOut));
+        bf16x4 d;
+        float e[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float out = y[r] + g.b4[4 * fg + r];
+            e[r] = live ? out - target[r] : 0.f;
+            d[r] = static_cast<__bf16>(scale * e[r]);
+            dyt[(4 * fg + r) * kTRow + srow] = d[r];
+        }
+        *reinterpret_cast<bf16x4*>(xs + srow * kXRow + 4 * fg) = d;
+        *reinterpret_cast<bf16x4*>(xs + srow * kXRow + kOut + 4 * fg) = bf16x4{};
+        // the row's loss: its sixteen outputs in order, across the four lanes that hold them
+        float l = 0.f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) l += e[r] * e[r];
+            l = __shfl(l, 16 * q + fr);
+        }
+        if (live && fg == 0) g.row_loss[r0 + srow] = l;
+    }
+    keep(f0, kHid, act + kActH3);
+    lds_barrier();
+    {
+        // b4: output t / 16 over the tile's 64 rows, by halves (32 apart, 16 apart, ... 1 apart)
+        const __bf16* row = dyt + (t >> 4) * kTRow + (t & 15);
+        float s = (static_cast<float>(row[0]) + static_cast<float>(row[32])) + (static_cast<float>(row[16]) + static_cast<float>(row[48]));
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) s += __shfl_xor(s, o);
+        if ((t & 15) == 0) bias_part[t >> 4] = s;
+    }
+    product(K1{}, xs, kXRow, acc);
+    weights(K4{}, g.W3t, kHid);
+    masked(acc, m3, sb, f1);
+    keep(dyt, kOut, act + kActDY);
+    lds_barrier();
+    product(K4{}, sb, kHRow, acc);
+    weights(K4{}, g.W2t, kHid);
+    masked(acc, m2, sa, f0);
+    keep(f1, kHid, act + kActG3);
+    bias_sums(f1, bias_part + kOut);
+    lds_barrier();
+    product(K4{}, sa, kHRow, acc);
+    masked(acc, m1, static_cast<__bf16*>(nullptr), f1);
+    keep(f0, kHid, act + kActG2);
+    bias_sums(f0, bias_part + kOut + kHid);
+    lds_barrier();
+    keep(f1, kHid, act + kActG1);
+    bias_sums(f1, bias_part + kOut + 2 * kHid);
+}
 
-    const int ntiles = (g.n + kFTile - 1) / kFTile;
-    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const int r0 = tile * kFTile;
-        __syncthreads();  // the previous tile's last reads of xt, gt and rows
-        if (t < kFTile) {
-            uint32_t row = uint32_t(min(r0 + t, g.n - 1));
-            if (g.st) row = g.idx[shuffle_index(epoch_pos + row, n_valid, g.half, key)];
-            rows[t] = row;
+// The weights' gradients of each split of the batch, dW[out x in] = sum of G[out, row] H[in, row], a
+// chain over the split's rows. Jobs 0, 1: halves of W3; 2, 3: of W2; 4: W1; 5: W4; a workgroup per job and
+// split, and the jobs of a split `splits` groups apart: with a multiple of eight of them on one XCD, whose
+// L2 then holds the split's rows. The groups after those sum 256 rows' losses per wave, and the rows'
+// b4 sums of their four tiles.
+struct WeightGradArgs {
+    int n, splits, per;  // rows, splits, rows per split
+    const __bf16* act;
+    const float *bias_part, *row_loss;
+    float* part;         // [splits x kGradTotal]
+    float* loss_part;    // [loss blocks]
+    float* b4_part;      // [loss blocks x kOut]
+};
+__global__ void __launch_bounds__(kFThreads, 2) mlp_weight_grad_kernel(WeightGradArgs g) {
+    const int t = threadIdx.x, w = t >> 6, lane = t & 63;
+    const int fr = lane & 15, fg = lane >> 4;
+    const int job = int(blockIdx.x) / g.splits, z = int(blockIdx.x) % g.splits;
+    if (job >= 6) {
+        const int b = 4 * (int(blockIdx.x) - 6 * g.splits) + w, first = b * kLossRows;
+        if (first >= g.n) return;
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = first + 64 * j + lane < g.n ? g.row_loss[first + 64 * j + lane] : 0.f;
+        float l = (v[0] + v[2]) + (v[1] + v[3]);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
+        if (lane == 0) g.loss_part[b] = l;
+        if (lane < kOut) {
+            const int tiles = (g.n + kFTile - 1) / kFTile;
+            float s = 0.f;
+            for (int k = 4 * b; k < min(4 * b + 4, tiles); ++k) s += g.bias_part[size_t(k) * kBiasCols + lane];
+            g.b4_part[size_t(b) * kOut + lane] = s;
         }
-        __syncthreads();
-        {
-            // thread t stages input features 2p, 2p + 1 (p = t % 16) of rows t / 16 + 16 j; rows past n
-            // and padding features are zero
-            const int p = t & 15, sr = t >> 4;
-            const bool in = 2 * p < kIn;
-            float2 v[kFTile / 16];
-#pragma unroll
-            for (int j = 0; j < kFTile / 16; ++j)
-                v[j] = *reinterpret_cast<const float2*>(g.X + size_t(rows[sr + 16 * j]) * kIn + (in ? 2 * p : 0));
-#pragma unroll
-            for (int j = 0; j < kFTile / 16; ++j) {
-                const int r = sr + 16 * j;
-                const bool live = in && r0 + r < g.n;
-                bf16x2 pv;
-                pv[0] = static_cast<__bf16>(live ? v[j].x : 0.f);
-                pv[1] = static_cast<__bf16>(live ? v[j].y : 0.f);
-                *reinterpret_cast<bf16x2*>(xs + r * kXRow + 2 * p) = pv;
-                xt[(2 * p) * kTRow + r] = pv[0];
-                xt[(2 * p + 1) * kTRow + r] = pv[1];
-            }
-        }
-        // the lane's four targets: outputs 4 fg.. of sample 16 w + fr
-        const int srow = 16 * w + fr;
-        const f32x4 target = *reinterpret_cast<const f32x4*>(g.T + size_t(rows[srow]) * kOut + 4 * fg);
-        __syncthreads();
-        const uint32_t m1 = forward(K1{}, xs, kXRow, g.W1, kInPad, c1, sa, h1t);
-        __syncthreads();
-        const uint32_t m2 = forward(K4{}, sa, kHRow, g.W2, kHid, c2, sb, h2t);
-        __syncthreads();
-        const uint32_t m3 = forward(K4{}, sb, kHRow, g.W3, kHid, c3, sa, h3t);
-        __syncthreads();
-        {
-            f32x4 y = c4;
-#pragma unroll
-            for (int kb = 0; kb < 4; ++kb)
-                y = mfma(*reinterpret_cast<const bf16x8*>(g.W4 + size_t(fr) * kHid + 32 * kb + fk),
-                         *reinterpret_cast<const bf16x8*>(sa + srow * kHRow + 32 * kb + fk), y);
-            const bool live = r0 + srow < g.n;
-            bf16x4 d;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float e = live ? y[r] - target[r] : 0.f;
-                loss += e * e;
-                d[r] = static_cast<__bf16>(scale * e);
-                db4[r] += static_cast<float>(d[r]);
-                dyt[(4 * fg + r) * kTRow + srow] = d[r];
-            }
-            *reinterpret_cast<bf16x4*>(dy + srow * kXRow + 4 * fg) = d;
-        }
-        __syncthreads();
-        backward(K1{}, dy, kXRow, g.W4t, kOutPad, m3, sb, gt, db3);
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {  // dW4[16 x 32w..32w+31]
-            const bf16x8 a = *reinterpret_cast<const bf16x8*>(dyt + fr * kTRow + 32 * kb + fk);
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-                dw4[b] = mfma(a, *reinterpret_cast<const bf16x8*>(h3t + (32 * w + 16 * b + fr) * kTRow + 32 * kb + fk), dw4[b]);
-        }
-        __syncthreads();
-        weight_grad(K8{}, gt, h2t, dw3);
-        backward(K4{}, sb, kHRow, g.W3t, kHid, m2, sa, h3t, db2);  // h3t now holds the second layer's gradient
-        __syncthreads();
-        weight_grad(K8{}, h3t, h1t, dw2);
-        backward(K4{}, sa, kHRow, g.W2t, kHid, m1, static_cast<__bf16*>(nullptr), gt, db1);
-        __syncthreads();
-        weight_grad(K2{}, gt, xt, dw1);
+        return;
     }
-    // the group's partial. D layout: the lane holds rows 4 fg + r of column fr of each 16 x 16 block
-    float* part = g.part + size_t(blockIdx.x) * kPartTotal;
+    const int kbeg = z * (g.per / kKStep), kend = min(g.n / kKStep, kbeg + g.per / kKStep);
+    float* part = g.part + size_t(z) * kGradTotal;
+    using N1 = std::integral_constant<int, 1>;
+    using N2 = std::integral_constant<int, 2>;
+    using N4 = std::integral_constant<int, 4>;
+    using N8 = std::integral_constant<int, 8>;
+    // dW[a .. a + 16 kA x b .. b + 16 kB] from the arrays at offA and offB
+    auto chain = [&](auto na, auto nb, int offA, int a, int offB, int b, float* dst, int ld) {
+        constexpr int kA = decltype(na)::value, kB = decltype(nb)::value;
+        f32x4 acc[kA][kB];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < kA; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int o = 32 * w + 16 * i + 4 * fg + r;
+            for (int c = 0; c < kB; ++c) acc[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+        auto blocks = [&](auto nu, int k0) {  // all loads in flight, then the products in order
+            constexpr int kU = decltype(nu)::value;
+            bf16x8 ga[kU][kA], hb[kU][kB];
 #pragma unroll
-            for (int b = 0; b < 8; ++b) {
-                part[kPartW3 + o * kHid + 16 * b + fr] = dw3[i][b][r];
-                part[kPartW2 + o * kHid + 16 * b + fr] = dw2[i][b][r];
+            for (int u = 0; u < kU; ++u) {
+                const __bf16* base = g.act + size_t((k0 + u) >> 1) * kActTile + 512 * ((k0 + u) & 1) + 8 * lane;
+#pragma unroll
+                for (int i = 0; i < kA; ++i) ga[u][i] = *reinterpret_cast<const bf16x8*>(base + offA + (a + 16 * i) * kFTile);
+#pragma unroll
+                for (int c = 0; c < kB; ++c) hb[u][c] = *reinterpret_cast<const bf16x8*>(base + offB + (b + 16 * c) * kFTile);
             }
+            __builtin_amdgcn_sched_barrier(0);  // the compiler would move each load to its product
 #pragma unroll
-            for (int b = 0; b < 2; ++b) part[kPartW1 + o * kInPad + 16 * b + fr] = dw1[i][b][r];
-            part[kPartW4 + (4 * fg + r) * kHid + 32 * w + 16 * i + fr] = dw4[i][r];
-        }
-    // bias sums over the 16 lanes of a feature (xor steps 1..8), in a fixed order
-    auto lanes16 = [](float v) {
+            for (int u = 0; u < kU; ++u)
 #pragma unroll
-        for (int o = 1; o < 16; o <<= 1) v += __shfl_xor(v, o);
-        return v;
+                for (int i = 0; i < kA; ++i)
+#pragma unroll
+                    for (int c = 0; c < kB; ++c) acc[i][c] = mfma(ga[u][i], hb[u][c], acc[i][c]);
+        };
+        int k = kbeg;
+        for (; k + 4 <= kend; k += 4) blocks(N4{}, k);
+        for (; k < kend; ++k) blocks(N1{}, k);
+        // D layout: the lane holds rows 4 fg + r of column fr of each 16 x 16 block
+#pragma unroll
+        for (int i = 0; i < kA; ++i)
+#pragma unroll
+            for (int c = 0; c < kB; ++c)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) dst[(a + 16 * i + 4 * fg + r) * ld + b + 16 * c + fr] = acc[i][c][r];
     };
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int f = 32 * w + 16 * i + 4 * fg + r;
-            const float s3 = lanes16(db3[i][r]), s2 = lanes16(db2[i][r]), s1 = lanes16(db1[i][r]);
-            if (fr == 0) {
-                part[kGradTotal + kOut + f] = s3;
-                part[kGradTotal + kOut + kHid + f] = s2;
-                part[kGradTotal + kOut + 2 * kHid + f] = s1;
-            }
-        }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const float s = lanes16(db4[r]);
-        if (fr == 0) red[w][1 + 4 * fg + r] = s;
-    }
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) loss += __shfl_xor(loss, o);
-    if (lane == 0) red[w][0] = loss;
-    __syncthreads();
-    if (t <= kOut) {
-        const float s = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
-        if (t == 0) g.loss_part[blockIdx.x] = s;
-        else part[kGradTotal + t - 1] = s;
+    if (job < 4) {
+        const bool third = job < 2;
+        chain(N1{}, N8{}, third ? kActG3 : kActG2, 64 * (job & 1) + 16 * w, third ? kActH2 : kActH1, 0, part + (third ? kPartW3 : kPartW2), kHid);
+    } else if (job == 4) {
+        chain(N2{}, N2{}, kActG1, 32 * w, kActX, 0, part + kPartW1, kInPad);
+    } else {
+        chain(N1{}, N2{}, kActDY, 0, kActH3, 32 * w, part + kPartW4, kHid);
     }
 }
-static_assert(sizeof(TrainState) <= kTrainStateWords * 4, "train state size");
 
-// Every gradient from the groups' partials, in one launch. A block takes 64 elements of a partial
-// with four threads each: thread group q sums the partials of groups q, q + 4, ... (16 loads issued
-// before their adds), and the four sums are combined in order. The sum goes to `grads`, or (grads
-// null) through Adam to the FP32 master parameters and their bf16 copies, whose padding stays zero;
-// the learning rate and the corrections come from the arguments, or with `st` from the device state
-// that the train kernel published. Block 0 then also records the step's mean loss and advances the
-// state's step, which no thread of this kernel reads.
+// Every gradient from its partial sums, in one launch. A weight has a partial per split, a hidden bias one
+// per tile, an output's bias one per 256 rows; four threads per element each add partials q, q + 4, ... in
+// order, and the four sums are combined in order. A block takes 64 weights, whose (at most 16) partials a
+// thread loads by itself, or 16 biases, whose many partials the block's threads stage 256 at a time.
+// The sum goes to `grads`, or (grads null) through Adam to the FP32 master parameters and their bf16
+// copies, whose padding stays zero; the learning rate and the corrections come from the arguments, or with
+// `st` from the device state that the train kernel published. Block 0 then also records the step's mean
+// loss, the losses' sums added in double in order, and advances the state's step, which no thread of this
+// kernel reads.
 struct WeightCopies {
-    __bf16 *W1, *W1t, *W2, *W2t, *W3, *W3t, *W4, *W4t;
+    __bf16 *W1, *W2, *W2t, *W3, *W3t, *W4, *W4t;
 };
 struct ReduceArgs {
-    int groups;
-    const float *part, *loss_part;
+    int splits, tiles, lblocks;
+    const float *part, *bias_part, *b4_part, *loss_part;
     float* grads;
     float *p, *m, *v;
     TrainState* st;
@@ -939,41 +1008,68 @@ struct ReduceArgs {
     WeightCopies w;
     float* loss_hist;
 };
-constexpr int kReduceLanes = 64, kReduceBatch = 16;  // elements per block; loads in flight per thread
+constexpr int kReduceLanes = 64, kReduceBias = 16;  // weights and biases per block
+constexpr int kWeightBlocks = kGradTotal / kReduceLanes, kReduceBlocks = kWeightBlocks + kBiasCols / kReduceBias;
+static_assert(kGradTotal % kReduceLanes == 0 && kBiasCols % kReduceBias == 0 && kOut == kReduceBias, "whole blocks");
 __global__ void __launch_bounds__(256) grad_reduce_kernel(ReduceArgs a) {
     __shared__ float sums[4][kReduceLanes];
-    const int el = threadIdx.x & (kReduceLanes - 1), q = threadIdx.x >> 6;
-    const int e = blockIdx.x * kReduceLanes + el;
-    const bool live = e < kPartTotal;
-    float acc = 0.f;
-    if (live) {
-        for (int z0 = q; z0 < a.groups; z0 += 4 * kReduceBatch) {
-            float v[kReduceBatch];
+    __shared__ float stage[256][kReduceBias];
+    const int t = threadIdx.x, block = int(blockIdx.x);
+    const bool bias = block >= kWeightBlocks;
+    if (!bias) {
+        const int el = t & (kReduceLanes - 1), q = t >> 6;
+        float v[kSplitTarget / 4], acc = 0.f;
 #pragma unroll
-            for (int j = 0; j < kReduceBatch; ++j) {
-                const int z = z0 + 4 * j;
-                v[j] = z < a.groups ? a.part[size_t(z) * kPartTotal + e] : 0.f;
+        for (int j = 0; j < kSplitTarget / 4; ++j) {
+            const int z = q + 4 * j;
+            v[j] = z < a.splits ? a.part[size_t(z) * kGradTotal + block * kReduceLanes + el] : 0.f;
+        }
+#pragma unroll
+        for (int j = 0; j < kSplitTarget / 4; ++j) acc += v[j];
+        sums[q][el] = acc;
+    } else {
+        const int first = (block - kWeightBlocks) * kReduceBias, el = t & (kReduceBias - 1), row = t / kReduceBias;
+        const float* src = (first == 0 ? a.b4_part : a.bias_part + first) + el;
+        const size_t stride = first == 0 ? kOut : kBiasCols;
+        const int count = first == 0 ? a.lblocks : a.tiles;
+        float acc = 0.f;
+        for (int z0 = 0; z0 < count; z0 += 256) {
+            float v[16];
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const int z = z0 + row + 16 * j;
+                v[j] = z < count ? src[size_t(z) * stride] : 0.f;
             }
 #pragma unroll
-            for (int j = 0; j < kReduceBatch; ++j) acc += v[j];
+            for (int j = 0; j < 16; ++j) stage[row + 16 * j][el] = v[j];
+            __syncthreads();
+            if (row < 4) {
+#pragma unroll 16
+                for (int j = 0; j < 64; ++j) acc += stage[row + 4 * j][el];
+            }
+            __syncthreads();
         }
+        if (row < 4) sums[row][el] = acc;
     }
-    sums[q][el] = acc;
     __syncthreads();
-    if (a.st && blockIdx.x == 0 && q == 1) {
+    if (a.st && block == 0 && t >= 64 && t < 128) {
+        const int el = t & 63;
         double l = 0.0;
-        for (int z = el; z < a.groups; z += kReduceLanes) l += double(a.loss_part[z]);
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) l += __shfl_xor(l, o);
+        for (int z0 = 0; z0 < a.lblocks; z0 += 64) {
+            const float v = z0 + el < a.lblocks ? a.loss_part[z0 + el] : 0.f;
+            const int m = min(64, a.lblocks - z0);
+            for (int k = 0; k < m; ++k) l += double(__shfl(v, k));
+        }
         if (el == 0) {
             const uint32_t now = a.st->now;
             a.loss_hist[now] = float(l / (double(a.st->batch) * kOut));
             a.st->step = now + 1u;
         }
     }
-    if (q != 0 || !live) return;
+    if (t >= (bias ? kReduceBias : kReduceLanes)) return;
+    const int el = t, e = bias ? kGradTotal + (block - kWeightBlocks) * kReduceBias + el : block * kReduceLanes + el;
     const float ge = (sums[0][el] + sums[1][el]) + (sums[2][el] + sums[3][el]);
-    // the element's parameter and, for a weight, its places in the two bf16 copies
+    // the element's parameter and, for a weight, its places in the bf16 copies
     size_t dst;
     __bf16 *W = nullptr, *Wt = nullptr;
     if (e < kPartW3) {
@@ -992,7 +1088,6 @@ __global__ void __launch_bounds__(256) grad_reduce_kernel(ReduceArgs a) {
         if (i >= kIn) return;  // padding
         dst = kOffW1 + size_t(o) * kIn + i;
         W = a.w.W1 + l;
-        Wt = a.w.W1t + i * kHid + o;
     } else {
         const int c = e - kGradTotal;
         dst = c < kOut ? kOffB4 + c : c < kOut + kHid ? kOffB3 + (c - kOut) : c < kOut + 2 * kHid ? kOffB2 + (c - kOut - kHid)
@@ -1013,31 +1108,34 @@ __global__ void __launch_bounds__(256) grad_reduce_kernel(ReduceArgs a) {
     if (W) {
         const __bf16 h = static_cast<__bf16>(pe);
         *W = h;
-        *Wt = h;
+        if (Wt) *Wt = h;
     }
 }
-WeightCopies weight_copies(const plt_surrogate* s) { return WeightCopies{s->W1, s->W1t, s->W2, s->W2t, s->W3, s->W3t, s->W4, s->W4t}; }
+WeightCopies weight_copies(const plt_surrogate* s) { return WeightCopies{s->W1, s->W2, s->W2t, s->W3, s->W3t, s->W4, s->W4t}; }
 
-int train_groups(uint32_t n) { return int(std::min<uint32_t>(kGroupsMax, (n + kFTile - 1) / kFTile)); }
-
-// The two launches of a step over n rows of X and T (with `st`, rows idx[shuffle]): the partials, then
-// their sums into `grads` or through Adam.
+// The launches of a step over n rows of X and T (with `st`, rows idx[shuffle]): the activations and
+// gradients, the splits' sums, then their sums into `grads` or through Adam.
 int train_launch(plt_surrogate* s, int n, const float* X, const float* T, const uint32_t* idx, int half, TrainState* st, float* grads, float lr,
                  float c1, float c2, float* loss_hist, hipStream_t qs) {
-    const int groups = train_groups(uint32_t(n));
+    const int tiles = tiles_of(uint32_t(n)), lblocks = loss_blocks(uint32_t(n));
+    const int per = split_len(uint32_t(n)), splits = (n + per - 1) / per;
     const TrainArgs ta{n, X, T, idx, half, st, s->W1, s->W2, s->W3, s->W4, s->W2t, s->W3t, s->W4t,
-                       s->params + kOffB1, s->params + kOffB2, s->params + kOffB3, s->params + kOffB4, s->part, s->loss_part};
-    hipLaunchKernelGGL(mlp_train_kernel, dim3(groups), dim3(kFThreads), 0, qs, ta);
+                       s->params + kOffB1, s->params + kOffB2, s->params + kOffB3, s->params + kOffB4, s->act, s->bias_part, s->row_loss};
+    hipLaunchKernelGGL(mlp_train_kernel, dim3(tiles), dim3(kFThreads), 0, qs, ta);
     int rc = check_launch("mlp_train_kernel");
     if (rc < 0) return rc;
-    const ReduceArgs ra{groups, s->part, s->loss_part, grads, s->params, s->adam_m, s->adam_v, st, lr, c1, c2, weight_copies(s), loss_hist};
-    hipLaunchKernelGGL(grad_reduce_kernel, dim3((kPartTotal + kReduceLanes - 1) / kReduceLanes), dim3(256), 0, qs, ra);
+    const WeightGradArgs wa{n, splits, per, s->act, s->bias_part, s->row_loss, s->part, s->loss_part, s->b4_part};
+    hipLaunchKernelGGL(mlp_weight_grad_kernel, dim3(6 * splits + (lblocks + 3) / 4), dim3(kFThreads), 0, qs, wa);
+    if ((rc = check_launch("mlp_weight_grad_kernel")) < 0) return rc;
+    const ReduceArgs ra{splits, tiles, lblocks, s->part, s->bias_part, s->b4_part, s->loss_part, grads, s->params, s->adam_m, s->adam_v, st, lr, c1,
+                        c2, weight_copies(s), loss_hist};
+    hipLaunchKernelGGL(grad_reduce_kernel, dim3(kReduceBlocks), dim3(256), 0, qs, ra);
     return check_launch("grad_reduce_kernel");
 }
 
 // The mean loss of the last train_launch over n rows.
 int read_loss(plt_surrogate* s, uint32_t n, float* loss, hipStream_t st) {
-    std::vector<float> lp(static_cast<size_t>(train_groups(n)));
+    std::vector<float> lp(static_cast<size_t>(loss_blocks(n)));
     if (hipMemcpyAsync(lp.data(), s->loss_part, lp.size() * sizeof(float), hipMemcpyDeviceToHost, st) != hipSuccess ||
         hipStreamSynchronize(st) != hipSuccess)
         return set_error(PLT_EHIP, "plt_surrogate: loss read-back failed");
@@ -1084,12 +1182,16 @@ int plt_surrogate_create(plt_context* ctx, uint32_t max_batch, uint32_t seed, pl
     int rc = PLT_OK;
     auto A = [&](auto** p, size_t count) { if (rc == PLT_OK) rc = dev_alloc(s, p, count); };
     A(&s->params, kParams); A(&s->grads, kParams); A(&s->adam_m, kParams); A(&s->adam_v, kParams);
-    A(&s->W1, size_t(kHid) * kInPad); A(&s->W1t, size_t(kInPad) * kHid);
+    A(&s->W1, size_t(kHid) * kInPad);
     A(&s->W2, size_t(kHid) * kHid); A(&s->W2t, size_t(kHid) * kHid);
     A(&s->W3, size_t(kHid) * kHid); A(&s->W3t, size_t(kHid) * kHid);
     A(&s->W4, size_t(kOut) * kHid); A(&s->W4t, size_t(kHid) * kOutPad);
-    A(&s->part, size_t(train_groups(max_batch)) * kPartTotal);
-    A(&s->loss_part, size_t(train_groups(max_batch)));
+    A(&s->act, size_t(tiles_of(max_batch)) * kActTile);
+    A(&s->bias_part, size_t(tiles_of(max_batch)) * kBiasCols);
+    A(&s->row_loss, max_batch);
+    A(&s->part, size_t(std::min(kSplitTarget, int(max_batch / kKStep))) * kGradTotal);
+    A(&s->loss_part, size_t(loss_blocks(max_batch)));
+    A(&s->b4_part, size_t(loss_blocks(max_batch)) * kOut);
     A(&s->train_state, kTrainStateWords);
     A(&s->stats, 2 * kOut + 2 * kIn);
     A(&s->counter, 1);

@@ -11,9 +11,12 @@ struct plt_surrogate {
     // FP32 master parameters (the public order), gradients, Adam moments
     float *params = nullptr, *grads = nullptr, *adam_m = nullptr, *adam_v = nullptr;
     uint32_t step = 0;
-    // bf16 operands: W (row-major [out x in_pad]) and Wt ([in x out_pad]) per layer
-    __bf16 *W1 = nullptr, *W1t = nullptr, *W2 = nullptr, *W2t = nullptr, *W3 = nullptr, *W3t = nullptr, *W4 = nullptr, *W4t = nullptr;
-    float *part = nullptr, *loss_part = nullptr;  // a training step's gradient and loss partials, one per workgroup
+    // bf16 operands: W (row-major [out x in_pad]) and, but for the first layer, Wt ([in x out_pad])
+    __bf16 *W1 = nullptr, *W2 = nullptr, *W2t = nullptr, *W3 = nullptr, *W3t = nullptr, *W4 = nullptr, *W4t = nullptr;
+    // a training step's activations and back-propagated gradients (per tile of 64 rows), bias sums (per
+    // tile), losses (per row), weight gradients (per split), and sums of losses and of b4 (per 256 rows)
+    __bf16* act = nullptr;
+    float *bias_part = nullptr, *row_loss = nullptr, *part = nullptr, *loss_part = nullptr, *b4_part = nullptr;
     uint32_t* train_state = nullptr;  // device-side training step state (plt_surrogate_train)
     // target statistics and the inputs' training box (plt_surrogate_set_stats): 16 + 16 + 22 + 22
     float* stats = nullptr;

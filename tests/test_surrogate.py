@@ -389,8 +389,8 @@ def test_gpu_surrogate_graph_training_equals_eager(gpu):
 @pytest.mark.parametrize("n", [32, 64, 96, 4128, 16448])
 def test_gpu_surrogate_fused_step_at_tile_edges(gpu, n):
     """Loss and gradients of batches around the training kernel's 64-row tiles (half a tile, one, one
-    and a half) and its 256 workgroups (65 tiles; 257, so one group takes two) against the restatement
-    with the same bf16 roundings. A sum in another order changes a result by FP32 rounding, or flips the
+    and a half) and the weight gradients' 64 splits (4,128: 43 of 96 rows, not whole tiles; 16,448: 52 of
+    320, the last one shorter) against the restatement with the same bf16 roundings. A sum in another order changes a result by FP32 rounding, or flips the
     bf16 rounding of an activation (a relative 2^-9 of it): 1e-3 of a tensor's norm allows a quarter of
     its activations to flip."""
     import torch
@@ -456,3 +456,80 @@ def test_gpu_surrogate_train_equals_steps_on_the_shuffled_rows(gpu, batch):
     print(f"batch {batch}: largest parameter difference {d:.2e}")
     assert d <= 1e-4 * lr * steps + 1e-7
     assert abs(runs[0][1] - runs[1][1]) <= 1e-5 * runs[1][1]
+
+
+def _grid_rows(n, seed):
+    """Inputs and targets on a grid of 2^-10, whatever the generator's floating-point path."""
+    rng = np.random.default_rng(seed)
+    return ((rng.integers(-1024, 1025, (n, 22)) / 1024).astype(np.float32), (rng.integers(-2048, 2049, (n, 16)) / 1024).astype(np.float32))
+
+
+# SHA-256 (first 16 digits) of the bits that the GEMM-per-product training path gave for these calls: loss
+# and gradients of a batch, and losses and weights after a training run.
+RECORDED_GRADIENTS = {32: "c30c04c4935655a3", 96: "437f8e0dc89bacd5", 160: "e395c538b90cf52a", 4128: "4fdac446780d4c45",
+                      6144: "6cc4f8b741b1dd8f", 16384: "d8e03adcb888ab26", 131072: "8178745ec4b8d557"}
+RECORDED_TRAINING = {9000: "37e8fa3f08aff6fc", 50000: "2b81ecac98d82736"}
+
+
+def _digest(*arrays):
+    import hashlib
+    h = hashlib.sha256()
+    for a in arrays:
+        h.update(np.ascontiguousarray(a, np.float32).tobytes())
+    return h.hexdigest()[:16]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [32, 96, 160, 4128, 6144, 16384, 131072])
+def test_gpu_surrogate_gradients_have_the_recorded_bits(gpu, n):
+    """Loss and gradients keep the order of their sums, whatever kernels compute them: blocks of 32 k, then
+    the bias; 64 splits of the batch; bias sums per 64 rows, losses per 256. The rows start one float into
+    their buffers: no wider alignment is asked of them."""
+    import torch
+    from pltfalcor_amd.surrogate import Surrogate
+    ctx, _ = _ctx_with_drude()
+    s = Surrogate(ctx, max_batch=n, seed=5)
+    s.set_params(R.he_init(n).astype(np.float32))
+    X, T = (torch.from_numpy(np.concatenate([np.zeros(1, np.float32), a.ravel()])).cuda()[1:].view(a.shape) for a in _grid_rows(n, n))
+    g, loss = s.gradients(X, T)
+    s.close()
+    assert _digest(g, [loss]) == RECORDED_GRADIENTS[n]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,batch", [(9000, 544), (50000, 6144)])
+def test_gpu_surrogate_training_has_the_recorded_bits(gpu, n, batch):
+    """The same for a training run from the targets' statistics on: column sums per 256 rows in row order,
+    the batches, Adam."""
+    import torch
+    from types import SimpleNamespace
+    from pltfalcor_amd.surrogate import Surrogate, train
+    ctx, _ = _ctx_with_drude()
+    s = Surrogate(ctx, max_batch=batch, seed=1)
+    s.set_params(R.he_init(3).astype(np.float32))
+    X, M = _grid_rows(n, batch)
+    M[:, 0] = np.abs(M[:, 0])  # some of them zero: rows that are not valid
+    losses = train(s, SimpleNamespace(n=n, X=torch.from_numpy(X).cuda(), M=torch.from_numpy(M).cuda()), epochs=2, batch=batch)
+    w = s.get_params()
+    s.close()
+    assert _digest(w, losses) == RECORDED_TRAINING[n]
+
+
+@pytest.mark.gpu
+def test_gpu_surrogate_loss_of_many_rows_keeps_small_terms(gpu):
+    """A batch of 2^20 rows whose first 16,384 errors are 4,096 and whose others are 1.97: the mean of the
+    squares needs every small one. Sixteen outputs and 256 rows are added in FP32 (at most 24 roundings of a
+    sum), everything above in double; one FP32 chain over a workgroup's tiles lost all of the small ones,
+    1.5e-5 of the result."""
+    import torch
+    from pltfalcor_amd.surrogate import Surrogate
+    ctx, _ = _ctx_with_drude()
+    n = 1 << 20
+    s = Surrogate(ctx, max_batch=n, seed=1)
+    s.set_params(np.zeros(R.N_PARAMS, np.float32))
+    e = np.full((n, 16), 1.97, np.float32)
+    e[:16384] = 4096
+    _, loss = s.gradients(torch.zeros((n, 22), device="cuda"), torch.from_numpy(e).cuda())
+    s.close()
+    ref = (e.astype(np.float64) ** 2).mean()
+    assert abs(loss - ref) <= 24 * 2.0 ** -24 * ref

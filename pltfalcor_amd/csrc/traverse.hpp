@@ -370,7 +370,8 @@ __device__ __forceinline__ Hit traverse(const TraceScene& sc, const Ray& r, int*
 }
 
 // ---------------------------------------------------------------------------------------
-// One ray per quad of lanes: lane i of the quad tests child i of a node and triangle i of a leaf.
+// One ray per quad of lanes: lane i of the quad tests child i of a node and triangles i and i + 4 of a
+// leaf (the host builder's have up to eight).
 // ---------------------------------------------------------------------------------------
 __device__ __forceinline__ uint32_t quad_xor1(uint32_t v) { return uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0xB1, 0xF, 0xF, true)); }
 __device__ __forceinline__ uint32_t quad_xor2(uint32_t v) { return uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0x4E, 0xF, 0xF, true)); }
@@ -437,6 +438,8 @@ __device__ __forceinline__ Hit traverse_quad(const TraceScene& sc, const Ray& r,
                 better(h, x);
                 if (anyHit) return h;
             }
+            next = (leaf & 4u) != 0u;  // more than four: the rest of the leaf is four triangles on, four fewer
+            node -= 28;                // = ~(leaf + 28)
         }
         if (!next) {
             if (sp == 0) break;

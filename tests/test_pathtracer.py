@@ -1266,3 +1266,111 @@ def test_gpu_split_solve_equals_megakernel(gpu, case):
                 print(f"{case['name']} {(ev, hits)} frame {f}: {int(diff.any(axis=2).sum())} pixels differ, max rel "
                       f"{rel.max():.3e}, quantiles 50/99 % of differing {np.quantile(rel[diff], [.5, .99])}")
             assert not diff.any(), (case["name"], ev, hits, f, int(diff.any(axis=2).sum()), np.argwhere(diff.any(axis=2))[:5])
+
+
+def _tubes_and_blades():
+    """The procedural scene with thin-walled tubes (diagonal 24-sided cylinders of long slivers) and clumps of
+    three crossed opaque quads: geometry whose host tree has leaves of five to eight triangles, where
+    splitting costs more than testing them, in both. Arrays (positions, normals, indices, tri_mesh,
+    mesh_material), materials, profiles, camera, and the tubes' and blades' material ids."""
+    from pltfalcor_amd import _lib
+    from pltfalcor_amd import materials as M
+    from pltfalcor_amd.scene import Scene
+    proc = Scene(None, seed=41, sphere_count=6, subdivision=2, material_kinds=8)
+    a = proc.numpy()
+    glass, blade = len(a["materials"]) // C.sizeof(_lib.Material), 0
+    parts = [[a[k]] for k in ("positions", "normals", "indices", "tri_mesh", "mesh_material")]
+    count = [len(a["positions"]), len(a["mesh_material"])]
+
+    def add(p, n, i, material):
+        for part, x in zip(parts, (np.asarray(p, np.float32), np.asarray(n, np.float32), np.asarray(i, np.uint32) + np.uint32(count[0]),
+                                   np.full(len(i), count[1], np.uint32), np.array([material], np.uint32))):
+            part.append(x)
+        count[0] += len(p)
+        count[1] += 1
+
+    rng = np.random.default_rng(2)
+    k = 24
+    i, phi = np.arange(k), 2 * np.pi * np.arange(k) / k
+    j = (i + 1) % k
+    for _ in range(12):
+        axis = np.array([rng.choice([-1, 1]), .6, rng.choice([-1, 1])]) * rng.uniform(.8, 1.2, 3)
+        axis /= np.linalg.norm(axis)
+        u = np.cross(axis, [0, 1, 0])
+        u /= np.linalg.norm(u)
+        n = np.cos(phi)[:, None] * u + np.sin(phi)[:, None] * np.cross(axis, u)
+        c = np.array([rng.uniform(-4, 4), 2.0, rng.uniform(-4, 4)])
+        add(np.concatenate([c - 2 * axis + .3 * n, c + 2 * axis + .3 * n]), np.concatenate([n, n]),
+            np.concatenate([np.stack([i, j, k + j], 1), np.stack([i, k + j, k + i], 1)]), glass)
+    for _ in range(60):
+        c = np.array([rng.uniform(-5, 5), .4, rng.uniform(-5, 5)])
+        for q in range(3):
+            th = np.pi * q / 3 + .1
+            d, up = np.array([np.cos(th), 0, np.sin(th)]) * .3, np.array([0, .4, 0])
+            add([c - d - up, c + d - up, c + d + up, c - d + up], [[-np.sin(th), 0, np.cos(th)]] * 4, [[0, 1, 2], [0, 2, 3]], blade)
+    return [np.concatenate(x) for x in parts], a["materials"] + M.pack([M.thin_dielectric(1.5, 1e-3)]), a["profiles"], proc.arrays.camera, glass, blade
+
+
+def _large_leaves(scene, arrays):
+    """Material ids of the leaves of more than four triangles."""
+    nodes, tris = scene.bvh_arrays()
+    refs = nodes[:, 24:28].view(np.int32)
+    leaf = ~refs[~np.isinf(nodes[:, 0:4]) & (refs < 0)]
+    first = tris[(leaf[(leaf & 7) > 3] >> 3), 0, 3].view(np.uint32)
+    return arrays[4][arrays[3][first]]
+
+
+def test_tubes_and_blades_have_large_leaves():
+    """The host builder ends at up to eight triangles where splitting them costs more."""
+    from pltfalcor_amd.scene import Scene
+    arrays, mats, profs, cam, glass, blade = _tubes_and_blades()
+    m = _large_leaves(Scene.from_arrays(None, *arrays, mats, profs, cam), arrays)
+    assert (m == glass).sum() > 50 and (m == blade).sum() > 20
+
+
+def _solve_frames(ctx, s, w, h, opts, frames=1, **cfg):
+    """Colours of a pass with this launch configuration, and its solve statistics (split schedule)."""
+    import torch
+    from pltfalcor_amd.pltpt import PLTPT
+    p = PLTPT(ctx, opts)
+    p.set_launch_config(**cfg)
+    p.set_scene(s)
+    out = []
+    color = torch.empty((h, w, 4), dtype=torch.float32, device="cuda")
+    albedo, normal = torch.empty_like(color), torch.empty_like(color)
+    for _ in range(frames):
+        color.fill_(float("nan"))
+        p.execute(w, h, color, albedo, normal)
+        torch.cuda.synchronize()
+        out.append(color.cpu().numpy().view(np.uint32).copy())
+    st = p.solve_stats() if cfg["solve_schedule"] == PLTPT.SOLVE_SPLIT else None
+    p.close()
+    return out, st
+
+
+@pytest.mark.gpu
+def test_gpu_walks_test_every_triangle_of_large_leaves(gpu):
+    """Manifold walks through and past leaves of five to eight triangles (the host builder's tree; the
+    device builder's leaves have at most four): with either tree the split pass, whose walks cast a ray
+    with four lanes, writes the megakernel's colour bit for bit, and its walks cast as many rays."""
+    from pltfalcor_amd.bsdf import default_context
+    from pltfalcor_amd.pltpt import PLTPT
+    from pltfalcor_amd.scene import Scene
+    ctx = default_context()
+    arrays, mats, profs, cam, _, _ = _tubes_and_blades()
+    opts = dict(BASE_OPTS, maxBounces=6, doMNEE=1)
+    frames, stats = [], []
+    for bvh in ("host", "device"):
+        s = Scene.from_arrays(ctx, *arrays, mats, profs, cam, bvh=bvh)
+        assert (len(_large_leaves(s, arrays)) > 0) == (bvh == "host")
+        frames.append(_solve_frames(ctx, s, 192, 128, opts, 2, solve_schedule=PLTPT.SOLVE_MEGAKERNEL)[0])
+        got, st = _solve_frames(ctx, s, 192, 128, opts, 2, solve_schedule=PLTPT.SOLVE_SPLIT)
+        print(bvh, st)
+        frames.append(got)
+        stats.append(st)
+        assert st["walks"] - st["failed_walks"] > 100 and st["overflowed_paths"] == 0
+    for k in range(1, 4):
+        for f in range(2):
+            diff = (frames[0][f] != frames[k][f]).any(axis=2)
+            assert not diff.any(), (k, f, int(diff.sum()), np.argwhere(diff)[:5])
+    assert stats[0] == stats[1]

@@ -226,6 +226,13 @@ int plt_material_eval_batch(plt_context* ctx, const plt_material* materials, uin
                             const float* queries, float* results, plt_stream stream);
 int plt_material_sample_batch(plt_context* ctx, const plt_material* materials, uint32_t n_materials, uint32_t n,
                               uint32_t frame, const float* queries, float* results, plt_stream stream);
+/* The same calls for a caller that knows its table: with PLT_MB_ONE_TYPE (all materials have one type) the
+ * queries are not ordered by type within the kernel's blocks. Only the time depends on it. */
+enum { PLT_MB_ONE_TYPE = 1 };
+int plt_material_eval_batch_ex(plt_context* ctx, const plt_material* materials, uint32_t n_materials, uint32_t n,
+                               const float* queries, float* results, uint32_t flags, plt_stream stream);
+int plt_material_sample_batch_ex(plt_context* ctx, const plt_material* materials, uint32_t n_materials, uint32_t n,
+                                 uint32_t frame, const float* queries, float* results, uint32_t flags, plt_stream stream);
 
 /* Pinhole camera (Scene/Camera/Camera.slang:46-78, Camera.cpp:187-193). */
 typedef struct plt_camera {

@@ -28,6 +28,7 @@ MQ_WI, MQ_WO, MQ_LOBE, MQ_MAT, MQ_LAMBDA, MQ_S, MQ_AREA, MQ_PLANES = 0, 3, 6, 7,
 MR_S, MR_PDF, MR_LAMBDA_PDF, MR_PLANES = 0, 16, 17, 21
 MSQ_WI, MSQ_MAT, MSQ_LAMBDA, MSQ_PLANES = 0, 3, 4, 5
 MSR_WO, MSR_PDF, MSR_WEIGHT, MSR_LOBE, MSR_VALID, MSR_PLANES = 0, 3, 4, 5, 6, 7
+MB_ONE_TYPE = 1
 
 
 class PLTError(RuntimeError):
@@ -125,6 +126,8 @@ SIGNATURES = [
     ("plt_scene_create_procedural", C.c_int, [C.c_void_p, C.POINTER(ProceduralSceneDesc), C.POINTER(C.c_void_p)]),
     ("plt_material_eval_batch", C.c_int, [C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint32, C.c_void_p, C.c_void_p,
                                           C.c_void_p]),
+    ("plt_material_eval_batch_ex", C.c_int, [C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint32, C.c_void_p, C.c_void_p,
+                                             C.c_uint32, C.c_void_p]),
     ("plt_pass_set_schedule", C.c_int, [C.c_void_p, C.c_int]),
     ("plt_pass_set_graph", C.c_int, [C.c_void_p, C.c_int]),
     ("plt_pass_set_launch_config", C.c_int, [C.c_void_p, C.POINTER(LaunchConfig)]),
@@ -156,6 +159,8 @@ SIGNATURES = [
     ("plt_mlp_gemm_nt", C.c_int, [C.c_uint32, C.c_uint32, C.c_uint32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),
     ("plt_material_sample_batch", C.c_int, [C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint32, C.c_uint32, C.c_void_p,
                                             C.c_void_p, C.c_void_p]),
+    ("plt_material_sample_batch_ex", C.c_int, [C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint32, C.c_uint32, C.c_void_p,
+                                               C.c_void_p, C.c_uint32, C.c_void_p]),
     ("plt_scene_create", C.c_int, [C.c_void_p, C.POINTER(SceneDesc), C.POINTER(C.c_void_p)]),
     ("plt_scene_create_ex", C.c_int, [C.c_void_p, C.POINTER(SceneDesc), C.c_int, C.POINTER(C.c_void_p),
                                       C.POINTER(BvhInfo)]),

@@ -98,12 +98,15 @@ def sample_generator_stream(n_streams: int, width: int, sample_number: int, draw
 
 class MaterialTable:
     """A device array of plt_material blocks for the batched material interface
-    (plt_material_eval_batch / plt_material_sample_batch)."""
+    (plt_material_eval_batch_ex / plt_material_sample_batch_ex)."""
 
     def __init__(self, ctx: Context, materials: bytes, device: str = "cuda"):
         self.ctx = ctx
         self.n = len(materials) // C.sizeof(_lib.Material)
-        self.data = torch.frombuffer(bytearray(materials), dtype=torch.uint8).to(device)
+        raw = bytearray(materials)
+        types = {m.type for m in (_lib.Material * self.n).from_buffer_copy(raw)}
+        self.flags = _lib.MB_ONE_TYPE if len(types) <= 1 else 0
+        self.data = torch.frombuffer(raw, dtype=torch.uint8).to(device)
 
     def eval(self, queries: torch.Tensor, stream=None) -> torch.Tensor:
         """queries: float32 [PLT_MQ_PLANES, n] on the device; returns [PLT_MR_PLANES, n]."""
@@ -112,9 +115,9 @@ class MaterialTable:
         q = queries.contiguous()
         n = q.shape[1]
         out = torch.empty((_lib.MR_PLANES, n), dtype=torch.float32, device=q.device)
-        _lib.check(_lib.load().plt_material_eval_batch(self.ctx.handle, C.c_void_p(self.data.data_ptr()), self.n, n,
-                                                       C.c_void_p(q.data_ptr()), C.c_void_p(out.data_ptr()),
-                                                       _stream_ptr(stream)))
+        _lib.check(_lib.load().plt_material_eval_batch_ex(self.ctx.handle, C.c_void_p(self.data.data_ptr()), self.n, n,
+                                                          C.c_void_p(q.data_ptr()), C.c_void_p(out.data_ptr()),
+                                                          self.flags, _stream_ptr(stream)))
         return out
 
     def sample(self, queries: torch.Tensor, frame: int = 0, stream=None) -> torch.Tensor:
@@ -125,7 +128,7 @@ class MaterialTable:
         q = queries.contiguous()
         n = q.shape[1]
         out = torch.empty((_lib.MSR_PLANES, n), dtype=torch.float32, device=q.device)
-        _lib.check(_lib.load().plt_material_sample_batch(self.ctx.handle, C.c_void_p(self.data.data_ptr()), self.n, n,
-                                                         frame, C.c_void_p(q.data_ptr()), C.c_void_p(out.data_ptr()),
-                                                         _stream_ptr(stream)))
+        _lib.check(_lib.load().plt_material_sample_batch_ex(self.ctx.handle, C.c_void_p(self.data.data_ptr()), self.n, n,
+                                                            frame, C.c_void_p(q.data_ptr()), C.c_void_p(out.data_ptr()),
+                                                            self.flags, _stream_ptr(stream)))
         return out

@@ -15,21 +15,33 @@ constexpr int kMatBlock = 256;
 // type, by whether the lobe is a delta, in a counting sort in LDS. Both kernels are bound by VALU issue,
 // and a wave of arbitrary queries ran every material's code in turn. Sorted, a wave spans three of ten
 // types; the planes' reads stay within the block's 1 KB of each. 200,003 eval queries over ten types:
-// 204 -> 99 us. Queries past n sort last. Every thread of the block calls it.
+// 172 -> 107 us. Queries past n sort last. Every thread of the block calls it. Blocks that need no order pay
+// for finding that out: 200,003 eval queries of one diffuse material 11.2 -> 11.9 us, of one thin dielectric
+// 25.1 -> 26.0 us; a table known to hold one type takes the kernels without it.
 __device__ uint32_t sorted_query(uint32_t n, const float* __restrict__ mat_plane, const float* __restrict__ lobe_plane,
                                  const plt_material* __restrict__ mats, uint32_t nmats) {
-    __shared__ uint32_t bins[64], order[kMatBlock];
+    __shared__ uint32_t bins[64], order[kMatBlock], differ[2][kMatBlock / 64];
     const uint32_t t = threadIdx.x, i = blockIdx.x * kMatBlock + t;
-    auto key_of = [&](uint32_t k) {
-        const uint32_t mi = __float_as_uint(mat_plane[k]);
-        uint32_t key = mi < nmats ? 2u * min(mats[mi].type, 30u) : 62u;
-        if (lobe_plane && (__float_as_uint(lobe_plane[k]) & kLobeDelta) != 0u) key |= 1u;
-        return min(key, 62u);
+    // whether any thread of the block says so: a vote per wave and one barrier
+    auto any = [&](int k, bool yes) {
+        const bool wave = __ballot(yes) != 0ull;
+        if ((t & 63u) == 0u) differ[k][t >> 6] = wave ? 1u : 0u;
+        __syncthreads();
+        uint32_t a = 0u;
+#pragma unroll
+        for (int w = 0; w < kMatBlock / 64; ++w) a |= differ[k][w];
+        return a != 0u;
     };
-    const uint32_t key = i < n ? key_of(i) : 63u;
-    // a block of one type keeps its order (a batch of one material, bound by memory, took a third longer
-    // with its lobes sorted)
-    if (__syncthreads_and((key >> 1) == (key_of(blockIdx.x * kMatBlock) >> 1) || i >= n)) return i;
+    const uint32_t first = __float_as_uint(mat_plane[blockIdx.x * kMatBlock]);
+    const uint32_t mine = i < n ? __float_as_uint(mat_plane[i]) : first;
+    // a block of one material keeps its order, which the index plane alone tells
+    if (!any(0, mine != first)) return i;
+    auto type_of = [&](uint32_t k) { return k < nmats ? min(mats[k].type, 30u) : 31u; };
+    const uint32_t type = type_of(mine);
+    // and a block of one type (bound by memory, it took a third longer with its lobes sorted)
+    if (!any(1, type != type_of(first))) return i;
+    const uint32_t delta = lobe_plane && i < n && (__float_as_uint(lobe_plane[i]) & kLobeDelta) != 0u ? 1u : 0u;
+    const uint32_t key = i < n ? min(2u * type + delta, 62u) : 63u;
     if (t < 64u) bins[t] = 0u;
     __syncthreads();
     const uint32_t rank = atomicAdd(&bins[key], 1u);
@@ -50,10 +62,12 @@ __device__ uint32_t sorted_query(uint32_t n, const float* __restrict__ mat_plane
     return order[t];
 }
 
+template <bool kSort>
 __global__ void __launch_bounds__(kMatBlock)
 material_eval_kernel(uint32_t n, const float* __restrict__ q, float* __restrict__ r, const plt_material* __restrict__ mats,
                      uint32_t nmats, const plt_spectral_profile* prof, uint32_t nprof) {
-    const uint32_t i = sorted_query(n, q + size_t(PLT_MQ_MAT) * n, q + size_t(PLT_MQ_LOBE) * n, mats, nmats);
+    const uint32_t i = kSort ? sorted_query(n, q + size_t(PLT_MQ_MAT) * n, q + size_t(PLT_MQ_LOBE) * n, mats, nmats)
+                             : blockIdx.x * kMatBlock + threadIdx.x;
     if (i >= n) return;
     auto Q = [&](int p) { return q[size_t(p) * n + i]; };
     const uint32_t mi = __float_as_uint(Q(PLT_MQ_MAT));
@@ -99,11 +113,12 @@ material_eval_kernel(uint32_t n, const float* __restrict__ q, float* __restrict_
     out[size_t(PLT_MR_PDF) * n] = mat_pdf(m, sd, wo, wi, beam.lambda[0]);
 }
 
+template <bool kSort>
 __global__ void __launch_bounds__(kMatBlock)
 material_sample_kernel(uint32_t n, uint32_t frame, const float* __restrict__ q, float* __restrict__ r,
                        const plt_material* __restrict__ mats, uint32_t nmats, const plt_spectral_profile* prof,
                        uint32_t nprof) {
-    const uint32_t i = sorted_query(n, q + size_t(PLT_MSQ_MAT) * n, nullptr, mats, nmats);
+    const uint32_t i = kSort ? sorted_query(n, q + size_t(PLT_MSQ_MAT) * n, nullptr, mats, nmats) : blockIdx.x * kMatBlock + threadIdx.x;
     if (i >= n) return;
     auto Q = [&](int p) { return q[size_t(p) * n + i]; };
     const uint32_t mi = __float_as_uint(Q(PLT_MSQ_MAT));
@@ -133,26 +148,36 @@ material_sample_kernel(uint32_t n, uint32_t frame, const float* __restrict__ q, 
 
 extern "C" {
 
-int plt_material_eval_batch(plt_context* ctx, const plt_material* materials, uint32_t n_materials, uint32_t n,
-                            const float* queries, float* results, plt_stream stream) {
-    if (!ctx || (n && (!queries || !results)) || (n_materials && !materials))
+int plt_material_eval_batch_ex(plt_context* ctx, const plt_material* materials, uint32_t n_materials, uint32_t n,
+                               const float* queries, float* results, uint32_t flags, plt_stream stream) {
+    if (!ctx || (n && (!queries || !results)) || (n_materials && !materials) || (flags & ~uint32_t(PLT_MB_ONE_TYPE)))
         return plt::set_error(PLT_EINVAL, "plt_material_eval_batch: bad arguments");
     if (n == 0) return PLT_OK;
-    hipLaunchKernelGGL(plt::material_eval_kernel, dim3((n + plt::kMatBlock - 1) / plt::kMatBlock), dim3(plt::kMatBlock), 0,
-                       static_cast<hipStream_t>(stream), n, queries, results, materials, n_materials, ctx->d_profiles,
-                       ctx->n_profiles);
+    const auto kernel = (flags & PLT_MB_ONE_TYPE) || n_materials <= 1 ? plt::material_eval_kernel<false> : plt::material_eval_kernel<true>;
+    hipLaunchKernelGGL(kernel, dim3((n + plt::kMatBlock - 1) / plt::kMatBlock), dim3(plt::kMatBlock), 0, static_cast<hipStream_t>(stream), n,
+                       queries, results, materials, n_materials, ctx->d_profiles, ctx->n_profiles);
     return plt::check_launch("material_eval_kernel");
+}
+
+int plt_material_eval_batch(plt_context* ctx, const plt_material* materials, uint32_t n_materials, uint32_t n,
+                            const float* queries, float* results, plt_stream stream) {
+    return plt_material_eval_batch_ex(ctx, materials, n_materials, n, queries, results, 0u, stream);
+}
+
+int plt_material_sample_batch_ex(plt_context* ctx, const plt_material* materials, uint32_t n_materials, uint32_t n, uint32_t frame,
+                                 const float* queries, float* results, uint32_t flags, plt_stream stream) {
+    if (!ctx || (n && (!queries || !results)) || (n_materials && !materials) || (flags & ~uint32_t(PLT_MB_ONE_TYPE)))
+        return plt::set_error(PLT_EINVAL, "plt_material_sample_batch: bad arguments");
+    if (n == 0) return PLT_OK;
+    const auto kernel = (flags & PLT_MB_ONE_TYPE) || n_materials <= 1 ? plt::material_sample_kernel<false> : plt::material_sample_kernel<true>;
+    hipLaunchKernelGGL(kernel, dim3((n + plt::kMatBlock - 1) / plt::kMatBlock), dim3(plt::kMatBlock), 0, static_cast<hipStream_t>(stream), n,
+                       frame, queries, results, materials, n_materials, ctx->d_profiles, ctx->n_profiles);
+    return plt::check_launch("material_sample_kernel");
 }
 
 int plt_material_sample_batch(plt_context* ctx, const plt_material* materials, uint32_t n_materials, uint32_t n,
                               uint32_t frame, const float* queries, float* results, plt_stream stream) {
-    if (!ctx || (n && (!queries || !results)) || (n_materials && !materials))
-        return plt::set_error(PLT_EINVAL, "plt_material_sample_batch: bad arguments");
-    if (n == 0) return PLT_OK;
-    hipLaunchKernelGGL(plt::material_sample_kernel, dim3((n + plt::kMatBlock - 1) / plt::kMatBlock), dim3(plt::kMatBlock),
-                       0, static_cast<hipStream_t>(stream), n, frame, queries, results, materials, n_materials,
-                       ctx->d_profiles, ctx->n_profiles);
-    return plt::check_launch("material_sample_kernel");
+    return plt_material_sample_batch_ex(ctx, materials, n_materials, n, frame, queries, results, 0u, stream);
 }
 
 }  // extern "C"

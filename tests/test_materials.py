@@ -504,3 +504,34 @@ def test_gpu_material_batches_do_not_depend_on_the_order_of_queries(gpu, n):
     short = table.sample(torch.from_numpy(q[:, :n].copy()).cuda(), frame=3).cpu().numpy()
     assert np.array_equal(long[:, :n].copy().view(np.uint32), short.view(np.uint32))
     assert np.all(long.view(np.uint32)[-1, b[_lib.MSQ_MAT] == len(mats)] == 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 256, 1000])
+def test_gpu_tables_of_one_type_skip_the_ordering(gpu, n):
+    """A table whose materials share a type takes the kernels that do not order queries: the same bits as
+    those queries give in a table of every type, a material index out of range among them."""
+    import torch
+    from pltfalcor_amd import _lib
+    from pltfalcor_amd import materials as M
+    from pltfalcor_amd.bsdf import MaterialTable, default_context
+    one = [M.thin_dielectric(1.5, .001, .1), M.thin_dielectric(1.4, .002, .05)]
+    mats = one + _all_materials()
+    uniform, mixed = (MaterialTable(default_context(), M.pack(x)) for x in (one, mats))
+    assert uniform.flags == _lib.MB_ONE_TYPE and mixed.flags == 0
+    rng = np.random.default_rng(n)
+    for planes, mat, run in ((_lib.MQ_PLANES, _lib.MQ_MAT, "eval"), (_lib.MSQ_PLANES, _lib.MSQ_MAT, "sample")):
+        q = rng.uniform(0.1, 1.0, (planes, n)).astype(np.float32)
+        q[0:3] /= np.linalg.norm(q[0:3], axis=0)
+        b = q.view(np.uint32)
+        if run == "eval":
+            q[3:6] = q[0:3] * np.array([[-1], [-1], [1]], np.float32)
+            b[_lib.MQ_LOBE] = rng.choice([0x04, 0x33, 0x40], n)
+            q[_lib.MQ_LAMBDA:_lib.MQ_LAMBDA + 4] = rng.uniform(380, 720, (4, n))
+        else:
+            q[_lib.MSQ_LAMBDA] = rng.uniform(380, 720, n)
+        b[mat] = rng.choice([0, 1, 2], n)
+        got = getattr(uniform, run)(torch.from_numpy(q.copy()).cuda()).cpu().numpy()
+        b[mat] = np.where(b[mat] == 2, len(mats), b[mat])
+        want = getattr(mixed, run)(torch.from_numpy(q.copy()).cuda()).cpu().numpy()
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), run

@@ -528,7 +528,7 @@ int plt_pass_execute(plt_pass* p, const plt_render_data* rd, plt_stream stream) 
     plt::camera_frame(s->host.camera, p->cam);
     plt::view_rotation(s->host.camera, p->view_rot);
     plt::PtScene sc{};
-    sc.tsc = plt::TraceScene{s->dev.nodes, s->dev.tris};
+    sc.tsc = plt::TraceScene{s->dev.nodes, s->dev.tris, s->dev.n_nodes};
     sc.positions = s->dev.positions;
     sc.normals = s->dev.normals;
     sc.indices = s->dev.indices;

@@ -393,7 +393,7 @@ int plt_scene_trace(plt_scene* scene, uint32_t n, const float* rays, uint32_t* h
         return set_error(PLT_EINVAL, "plt_scene_trace: bad arguments");
     if (!scene->ctx) return set_error(PLT_ESTATE, "plt_scene_trace: host-only scene (created without a context)");
     if (n == 0) return PLT_OK;
-    plt::TraceScene sc{scene->dev.nodes, scene->dev.tris};
+    plt::TraceScene sc{scene->dev.nodes, scene->dev.tris, scene->dev.n_nodes};
     const dim3 grid((n + plt::kTraceBlock - 1) / plt::kTraceBlock), block(plt::kTraceBlock);
     if (mode == 0)
         hipLaunchKernelGGL(plt::trace_kernel<false>, grid, block, 0, static_cast<hipStream_t>(stream), sc, n, rays, hits);

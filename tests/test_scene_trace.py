@@ -120,6 +120,22 @@ def test_gpu_trace_bit_exact_path_scene(gpu):
         assert (g[0] != 0xFFFFFFFF).mean() > 0.3
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("spheres,small", [(1, True), (64, True), (100, False)])
+def test_gpu_trace_bit_exact_on_both_sides_of_the_small_tree_rule(gpu, spheres, small):
+    """Trees of fewer than 4,096 nodes cast closest hits with another loop than larger ones; any-hit rays
+    keep theirs. Both give the oracle's hits."""
+    import torch
+    ctx, s = _gpu_scene(seed=7, sphere_count=spheres, subdivision=2)
+    assert (s.bvh_info()["n_nodes"] < 4096) == small
+    a = s.numpy()
+    for rays in (random_rays(20000, 8), edge_rays(a), random_rays(3, 9)):
+        g = s.trace(torch.from_numpy(rays).cuda()).cpu().numpy().view(np.uint32)
+        assert np.array_equal(g, O.trace(a["positions"], a["indices"], rays))
+        ga = s.trace(torch.from_numpy(rays).cuda(), any_hit=True).cpu().numpy()
+        assert np.array_equal(ga.astype(np.uint32), O.trace(a["positions"], a["indices"], rays, any_hit=True))
+
+
 def test_scene_from_arrays_matches_procedural():
     """plt_scene_create from caller arrays reproduces the procedural scene (same arrays, and the
     oracle's intersections with rays agree for both), and rejects out-of-range ids."""

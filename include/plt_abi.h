@@ -339,8 +339,12 @@ typedef struct plt_bvh_info {
 /* Rebuilds the tree of a scene created with a context and replaces the one it holds (after waiting
  * for the device: passes bound to the scene read the tree at their next execute). The device
  * builder runs on `stream` and synchronizes it. PLT_EINVAL when the device tree would need more
- * levels than the traversal stack holds (33); the scene then keeps its tree. */
+ * levels than the traversal stack holds (33); the scene then keeps its tree.
+ * After a device build the scene keeps the builder's scratch memory (about 300 B per triangle) and the
+ * buffers of the tree before it (about 70 B per triangle) for the next one; a host build, a failed
+ * build, plt_scene_release_build_memory and plt_scene_destroy give them back. Creating a scene keeps none. */
 int plt_scene_build_bvh(plt_scene* scene, int builder, plt_stream stream, plt_bvh_info* info);
+int plt_scene_release_build_memory(plt_scene* scene);
 /* plt_scene_create with a choice of builder: PLT_BVH_DEVICE_PLOC builds no host tree (it falls
  * back to the host builder if the device tree would be too deep; info->builder says which ran).
  * ctx must not be NULL for the device builder. info may be NULL. */

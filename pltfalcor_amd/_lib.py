@@ -165,6 +165,7 @@ SIGNATURES = [
     ("plt_scene_create_ex", C.c_int, [C.c_void_p, C.POINTER(SceneDesc), C.c_int, C.POINTER(C.c_void_p),
                                       C.POINTER(BvhInfo)]),
     ("plt_scene_build_bvh", C.c_int, [C.c_void_p, C.c_int, C.c_void_p, C.POINTER(BvhInfo)]),
+    ("plt_scene_release_build_memory", C.c_int, [C.c_void_p]),
     ("plt_scene_get_bvh", C.c_int, [C.c_void_p, C.POINTER(BvhInfo), C.c_void_p, C.c_size_t, C.c_void_p, C.c_size_t]),
     ("plt_scene_destroy", C.c_int, [C.c_void_p]),
     ("plt_scene_get_arrays", C.c_int, [C.c_void_p, C.POINTER(SceneArrays)]),

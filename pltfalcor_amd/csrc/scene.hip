@@ -130,15 +130,19 @@ void host_bvh_info(const HostScene& hs, plt_bvh_info& info) {
     info.build_ms = hs.bvh.build_ms;
 }
 
-// Builds the scene's tree on the device and installs it; the scene keeps its old tree on failure. The
-// old tree's buffers go to the scene's build workspace.
+// Builds the scene's tree on the device and installs it; the scene keeps its old tree on failure, and
+// gives its build workspace back. The old tree's buffers go to that workspace.
 int device_bvh(plt_scene* s, hipStream_t st) {
     DeviceBvh b;
     const int rc = build_bvh_device(s->dev, st, s->work, b);
-    if (rc < 0) return rc;
+    if (rc < 0) {
+        s->work.release();
+        return rc;
+    }
     if (hipDeviceSynchronize() != hipSuccess) {
         (void)hipFree(b.nodes);
         (void)hipFree(b.tris);
+        s->work.release();
         return set_error(PLT_EHIP, "device BVH build: device synchronization failed");
     }
     auto swap_owned = [&](float4* old, float4* now) {  // false: the scene held none
@@ -284,6 +288,7 @@ int plt_scene_build_bvh(plt_scene* scene, int builder, plt_stream stream, plt_bv
         if (rc < 0) return rc;
     } else {
         plt::HostBvh b = plt::build_bvh(h.positions, h.indices, 4);
+        scene->work.release();  // the device builder's
         if (scene->ctx) {
             if (hipDeviceSynchronize() != hipSuccess) return set_error(PLT_EHIP, "plt_scene_build_bvh: device synchronization failed");
             std::swap(h.bvh, b);
@@ -298,6 +303,12 @@ int plt_scene_build_bvh(plt_scene* scene, int builder, plt_stream stream, plt_bv
         plt::host_bvh_info(h, scene->bvh);
     }
     if (info) *info = scene->bvh;
+    return PLT_OK;
+}
+
+int plt_scene_release_build_memory(plt_scene* scene) {
+    if (!scene) return set_error(PLT_EINVAL, "plt_scene_release_build_memory: NULL scene");
+    scene->work.release();
     return PLT_OK;
 }
 

@@ -117,7 +117,8 @@ class Scene:
     def build_bvh(self, builder: str = "device", stream=None) -> dict:
         """Rebuilds the scene's BVH with the host ("host") or device ("device") builder and returns
         bvh_info(). A device tree deeper than the traversal stack holds raises (PLT_EINVAL) and the
-        scene keeps its tree."""
+        scene keeps its tree. A device build's working memory (about 370 B per triangle) stays with
+        the scene for the next one until release_build_memory() or a host build."""
         if stream is None and self.ctx is not None and torch.cuda.is_available():
             stream = torch.cuda.current_stream()
         info = _lib.BvhInfo()
@@ -126,6 +127,10 @@ class Scene:
                                                 C.byref(info)))
         self._refresh_arrays()
         return self.bvh_info()
+
+    def release_build_memory(self):
+        """Gives back what device builds keep between them (after the last build_bvh of a scene)."""
+        _lib.check(self.lib.plt_scene_release_build_memory(self.handle))
 
     def bvh_info(self) -> dict:
         info = _lib.BvhInfo()

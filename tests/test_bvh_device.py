@@ -306,3 +306,31 @@ def test_gpu_rebuilds_reuse_the_scenes_buffers(gpu, n):
         nodes, tris = s.bvh_arrays()
         check_tree(nodes, tris, pos, idx)
         _trace_both(s, pos, idx, random_rays(1000, n, lo=-12, hi=12))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("give_back", ["host build", "release"])
+def test_gpu_scene_gives_its_build_memory_back(gpu, give_back):
+    """Device rebuilds keep their working memory with the scene; a host build and an explicit release
+    return it, and the scene casts and rebuilds as before."""
+    import torch
+    from pltfalcor_amd.bsdf import Context
+    ctx = Context(0)
+    a, base, pos, nrm, idx = _soup(300_000, seed=5)
+    s = _from(ctx, a, base, pos, nrm, idx, "host")
+    used = lambda: torch.cuda.mem_get_info()[1] - torch.cuda.mem_get_info()[0]  # noqa: E731
+    before = used()
+    for _ in range(2):
+        s.build_bvh("device")
+    assert used() - before > 250 * len(idx)  # scratch and a second tree
+    if give_back == "release":
+        s.release_build_memory()
+    else:
+        s.build_bvh("host")
+    # the trees' sizes differ a little; allocations are rounded up
+    assert used() - before < 60 * len(idx) + (4 << 20)
+    s.build_bvh("device")
+    check_tree(*s.bvh_arrays(), pos, idx)
+    s.release_build_memory()
+    s.release_build_memory()
+    _trace_both(s, pos, idx, random_rays(200, 3, lo=-12, hi=12))

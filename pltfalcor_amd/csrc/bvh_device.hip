@@ -50,9 +50,6 @@ constexpr uint32_t kLeafMax = 4;          // triangles per leaf at most
 // geometry that merges only a few per iteration, such as sizes growing geometrically, would also
 // make a tree too deep for the traversal stack).
 constexpr int kMaxIterations = 4096;
-// Levels of 4-wide nodes at most: every level on the way down pushes up to three stack entries.
-constexpr int kMaxLevels = 33;
-static_assert(3 * kMaxLevels <= kTraversalStackDepth + kTraversalSpill, "the traversal stack holds the deepest tree");
 
 // Spreads the low 21 bits of v to every third bit.
 __device__ __forceinline__ uint64_t spread3(uint32_t v) {
@@ -678,8 +675,8 @@ int build_bvh_device(const DeviceSceneBuffers& d, hipStream_t st, BvhWork& work,
     int levels = 0;
     std::vector<uint32_t> level_first, level_width;
     while (width > 0) {
-        if (levels == kMaxLevels)
-            return set_error(PLT_EINVAL, "device BVH build: the tree needs more than " + std::to_string(kMaxLevels) +
+        if (levels == kMaxTreeLevels)
+            return set_error(PLT_EINVAL, "device BVH build: the tree needs more than " + std::to_string(kMaxTreeLevels) +
                                              " levels of 4-wide nodes, more than the traversal stack holds");
         if (hipMemsetAsync(next_count, 0, 4, st) != hipSuccess) return hip_fail("collapse");
         hipLaunchKernelGGL(collapse_kernel, dim3(grid_of(width)), dim3(kBlock), 0, st, width, items, level_base, next,

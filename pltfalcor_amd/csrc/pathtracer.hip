@@ -240,8 +240,10 @@ int launch_solve_pass(const PtScene& sc, const PtFrame& fr, hipStream_t st) {
     return set_error(PLT_ENOTIMPL, "HWSS sample counts other than 1 and 4 are not built");
 }
 
-// Split solve pass: light sampling, unwind, then the megakernel over the paths whose region's event
-// area overflowed (its other blocks return at once). Three launches on one stream, no host waits.
+// Split solve pass: light sampling, the manifold walks with the unwind of the other events beside them on
+// the second stream, the walks' unwind and the sums (with a surrogate: the walks, then its passes, on one
+// stream), then the megakernel over the paths whose region's event area overflowed (its other blocks
+// return at once). No host waits.
 int launch_solve_pass_split(const PtScene& sc, const PtFrame& fr, const SolveBuffers& sb, hipStream_t st, hipEvent_t after_light,
                             hipEvent_t after_walk, hipEvent_t after_unwind, plt_surrogate* surrogate, const SplitFork& fork) {
     if (fr.n_paths == 0) {
@@ -269,15 +271,14 @@ int launch_solve_pass_split(const PtScene& sc, const PtFrame& fr, const SolveBuf
         // The walk kernel's last walks keep a few waves busy for long: the events that are
         // not walks are unwound beside it on the second stream (their contributions stored), the
         // walks that succeeded after it, and then every path's contributions are summed in order.
-        const hipStream_t side = fork.aux ? fork.aux : st;
-        if (fork.aux && (hipEventRecord(fork.fork, st) != hipSuccess || hipStreamWaitEvent(fork.aux, fork.fork, 0) != hipSuccess))
+        if (hipEventRecord(fork.fork, st) != hipSuccess || hipStreamWaitEvent(fork.aux, fork.fork, 0) != hipSuccess)
             return set_error(PLT_EHIP, "split solve pass: fork to the second stream failed");
-        if ((rc = launch_solve_unwind(sc, fr, sb, side)) < 0) return rc;
-        if (fork.aux && hipEventRecord(fork.join, fork.aux) != hipSuccess) return set_error(PLT_EHIP, "split solve pass: join event failed");
+        if ((rc = launch_solve_unwind(sc, fr, sb, fork.aux)) < 0) return rc;
+        if (hipEventRecord(fork.join, fork.aux) != hipSuccess) return set_error(PLT_EHIP, "split solve pass: join event failed");
         if ((rc = launch_solve_walks(sc, fr, sb, st)) < 0) return rc;
         if (after_walk) (void)hipEventRecord(after_walk, st);
         if ((rc = launch_solve_walk_unwind(sc, fr, sb, st)) < 0) return rc;
-        if (fork.aux && hipStreamWaitEvent(st, fork.join, 0) != hipSuccess) return set_error(PLT_EHIP, "split solve pass: join failed");
+        if (hipStreamWaitEvent(st, fork.join, 0) != hipSuccess) return set_error(PLT_EHIP, "split solve pass: join failed");
         if ((rc = launch_solve_sum(fr, sb, st)) < 0) return rc;
     }
     if (after_unwind) (void)hipEventRecord(after_unwind, st);

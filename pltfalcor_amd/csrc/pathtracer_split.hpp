@@ -12,15 +12,18 @@
 // visibility and completes the event or voids it. It holds the traversal stack but no beam and no
 // BSDF evaluation.
 //
-// solve_unwind_kernel rebuilds each event's beam and runs the rest of the megakernel's sequence
+// The unwind kernels rebuild each event's beam and run the rest of the megakernel's sequence
 // for it -- MIS weight, walk unwind (manifoldForwardUnwind, :80-93), evalNEE (:219-243),
-// forwardUnwind (:48-79), measure (:96-147) -- and sums each path's contributions in the order the
+// forwardUnwind (:48-79), measure (:96-147): solve_unwind_staged_kernel for the events that are not
+// walks, beside the walk kernel, solve_walk_unwind_kernel for the walks that succeeded. They store an
+// event's contribution in its slot, and solve_sum_kernel adds each path's contributions in the order the
 // megakernel adds them (the events of a path are stored in its own vertex order), so the colour is
-// the megakernel's bit for bit. It holds the beam and the material evaluations but no traversal.
+// the megakernel's bit for bit. They hold the beam and the material evaluations but no traversal.
+// With a surrogate, solve_unwind_kernel does all of this in its query and apply passes.
 //
 // A region (64 consecutive paths, one wave) has room for 64 * ev_per_path events and 64 *
 // hits_per_path walk vertices. A path whose events do not fit is flagged in the region's overflow
-// mask; the unwind kernel skips it and the megakernel, launched after it with the mask, solves it.
+// mask; the unwind kernels skip it and the megakernel, launched after it with the mask, solves it.
 #pragma once
 #include "pathtracer_kernels.hpp"
 #include "surrogate_features.hpp"
@@ -37,8 +40,8 @@ PLT_DEV void ev_put3(const SolveBuffers& sb, size_t e, int f, V3 v) {
     ev_putf(sb, e, f + 1, v.y);
     ev_putf(sb, e, f + 2, v.z);
 }
-// Event and bounce-record reads are non-temporal: each word is read once, by the unwind kernels,
-// which run beside the walk kernel on a second stream. Measured per 1080p frame of the
+// Event and bounce-record reads are non-temporal: each word is read once, by the unwind kernels (whose sort
+// looks at an event's first word twice before, with plain loads), which run beside the walk kernel on a second stream. Measured per 1080p frame of the
 // 5.24M-triangle scene (mean of three interleaved runs): walk kernel 3.54 -> 3.47 ms with its L2
 // fetch unchanged; the staged unwind's fetch rose 7.6 % and its writes fell 10 %.
 PLT_DEV uint32_t ev_get(const SolveBuffers& sb, size_t e, int f) { return __builtin_nontemporal_load(sb.ev + size_t(f) * sb.ev_cap + e); }

@@ -69,10 +69,10 @@ void replace_owned(DeviceSceneBuffers& d, void* old, void* now) {
 // Uploads the host tree: nodes as float4 x 8 and triangles in leaf order as (v0, id), (v1, 0),
 // (v2, 0), replacing the tree the scene holds.
 int upload_bvh(const HostScene& hs, DeviceSceneBuffers& d) {
-    // a BVH4 of L levels pushes at most 3 L entries; the builder's depth bound keeps L <= 32
-    if (3 * hs.bvh.max_depth > kTraversalStackDepth + kTraversalSpill)
+    // the builder's depth bound keeps the levels at 32
+    if (hs.bvh.max_depth > kMaxTreeLevels)
         return set_error(PLT_EINVAL, "BVH depth " + std::to_string(hs.bvh.max_depth) + " exceeds the traversal stack (" +
-                                         std::to_string(kTraversalStackDepth + kTraversalSpill) + " entries)");
+                                         std::to_string(kMaxTreeLevels) + " levels)");
     std::vector<float4> nodes(hs.bvh.nodes.size() * 8);
     std::memcpy(nodes.data(), hs.bvh.nodes.data(), hs.bvh.nodes.size() * sizeof(BvhNode));
     const size_t nt = hs.bvh.tri_order.size();

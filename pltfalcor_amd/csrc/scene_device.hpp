@@ -8,10 +8,6 @@
 
 namespace plt {
 
-// Traversal stack entries kept in LDS per lane; deeper entries go to private memory (traverse.hpp).
-// 32 slots x 4 B x 64 lanes = 8 KB per one-wave block, which leaves LDS room for 20 blocks per CU.
-constexpr int kTraversalStackDepth = 32;
-
 struct DeviceSceneBuffers {
     float4* nodes = nullptr;          // 8 x float4 per BVH node (BvhNode, 128 B)
     float4* tris = nullptr;           // 3 x float4 per triangle, leaf order (48 B)

@@ -94,9 +94,14 @@ __device__ __forceinline__ bool intersect_tri(const RayPrep& p, float4 v0, float
     return true;
 }
 
-// Entries of the traversal stack beyond the LDS part, in private memory. Every node on the way down
-// pushes at most three children, so a tree of 33 levels (the most the builders make) needs 99 entries.
+// Levels of 4-wide nodes that a scene's tree may have: the device builder and the upload of a host tree
+// refuse more. Every node on the way down pushes at most three children.
+constexpr int kMaxTreeLevels = 33;
+// Traversal stack entries kept in LDS per lane (32 slots x 4 B x 64 lanes = 8 KB per one-wave block, which
+// leaves LDS room for 20 blocks per CU), and the entries beyond them, in private memory.
+constexpr int kTraversalStackDepth = 32;
 constexpr int kTraversalSpill = 68;
+static_assert(3 * kMaxTreeLevels <= kTraversalStackDepth + kTraversalSpill, "the traversal stack holds the deepest tree");
 
 // Sorts four keys ascending (five compare-exchanges).
 __device__ __forceinline__ void sort4(uint32_t& a, uint32_t& b, uint32_t& c, uint32_t& d) {
@@ -385,9 +390,9 @@ __device__ __forceinline__ uint32_t quad_xor1(uint32_t v) { return uint32_t(__bu
 __device__ __forceinline__ uint32_t quad_xor2(uint32_t v) { return uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0x4E, 0xF, 0xF, true)); }
 __device__ __forceinline__ uint32_t quad_xor3(uint32_t v) { return uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0x1B, 0xF, 0xF, true)); }
 __device__ __forceinline__ uint32_t quad_first(uint32_t v) { return uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0x00, 0xF, 0xF, true)); }
-// Stack entries of a quad's traversal, all in LDS: three for each of the 33 levels of the deepest tree
-// the builders make, interleaved over the wave's 16 quads ([entry][quad]).
-constexpr int kQuadStack = 100;
+// Stack entries of a quad's traversal, all in LDS, interleaved over the wave's 16 quads ([entry][quad]).
+// Its pushes are not checked.
+constexpr int kQuadStack = 3 * kMaxTreeLevels;
 constexpr int kQuads = 16;
 
 // The hit traverse_rays finds for the same ray, cast by the four lanes of a quad together (the ray is

@@ -11,7 +11,7 @@ import oracle_lib as O
 from test_pathtracer import _path_len
 from test_scene_trace import _staircase, edge_rays, random_rays
 
-MAX_LEVELS = 33  # 3 (levels - 1) traversal stack entries <= 32 in LDS + 64 spilled
+MAX_LEVELS = 33  # 3 entries a level: 99 of the traversal stack's 32 in LDS + 68 spilled
 
 
 def check_tree(nodes, tris, pos, idx):

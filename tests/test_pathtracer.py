@@ -1374,3 +1374,74 @@ def test_gpu_walks_test_every_triangle_of_large_leaves(gpu):
             diff = (frames[0][f] != frames[k][f]).any(axis=2)
             assert not diff.any(), (k, f, int(diff.sum()), np.argwhere(diff)[:5])
     assert stats[0] == stats[1]
+
+
+def _deep_sheet_scene(ctx):
+    """A thin dielectric sheet under a distant light, and beside it a staircase of 300 triangles whose sizes grow
+    geometrically (a chain of 19 levels). The light's direction passes inside every step's box and past its
+    triangle, so a ray towards it leaves siblings on the stack at every level."""
+    from pltfalcor_amd import materials as M
+    from pltfalcor_amd.lights import DistantLight
+    from pltfalcor_amd.scene import Scene
+    mats = [M.diffuse(.5, .5, .5), M.diffuse(.8, .8, .8, emission=2), M.thin_dielectric(1.5, 1e-3)]
+    a = _look_down(_quad_scene([(0.0, 10.0, 1.0, 0), (-50.0, 1.0, -1.0, 1), (1.5, 10.0, 1.0, 2)], mats), height=0.6)
+    n, nv = 300, len(a["positions"])
+    x = (30 * 1.1 ** np.arange(n)).astype(np.float32)
+    step = np.stack([np.stack([x, 0 * x, 0 * x], 1), np.stack([x, 2.5 * x, 0 * x], 1), np.stack([x, 0 * x, 1.2 * x], 1)], 1)
+    s = Scene.from_arrays(ctx, np.concatenate([a["positions"], step.reshape(-1, 3)]),
+                          np.concatenate([a["normals"], np.tile(np.float32([-1, 0, 0]), (3 * n, 1))]),
+                          np.concatenate([a["indices"], nv + np.arange(3 * n, dtype=np.uint32).reshape(n, 3)]),
+                          np.concatenate([a["tri_mesh"], np.full(n, a["tri_mesh"].max() + 1, np.uint32)]),
+                          np.concatenate([a["mesh_material"], np.zeros(1, np.uint32)]), a["materials"], a["profiles"], _camera_struct(a["camera"]))
+    sun = DistantLight()
+    sun.direction = (-1.0, -2.0, -0.9)
+    sun.setIntensity(2)
+    if ctx is not None:
+        s.set_lights([sun])
+    return s
+
+
+def test_deep_sheet_scene_is_deep():
+    assert _deep_sheet_scene(None).bvh_info()["max_depth"] >= 16
+
+
+@pytest.mark.gpu
+def test_gpu_walks_through_a_deep_tree(gpu):
+    """Walks whose rays hold a deep stack, all of it in the quad's LDS: the megakernel's colour bit for bit."""
+    from pltfalcor_amd.bsdf import default_context
+    from pltfalcor_amd.pltpt import PLTPT
+    ctx = default_context()
+    s = _deep_sheet_scene(ctx)
+    opts = dict(BASE_OPTS, maxBounces=3, doMNEE=1)
+    ref, _ = _solve_frames(ctx, s, 96, 64, opts, solve_schedule=PLTPT.SOLVE_MEGAKERNEL)
+    got, st = _solve_frames(ctx, s, 96, 64, opts, solve_schedule=PLTPT.SOLVE_SPLIT)
+    print(st)
+    assert st["walks"] - st["failed_walks"] > 1000
+    assert np.array_equal(ref[0], got[0])
+
+
+@pytest.mark.gpu
+def test_gpu_unwind_sorts_more_events_than_its_list_holds(gpu):
+    """Blocks of several regions with more than the 4,096 events that are sorted at a time, of every light
+    type and walks among them: the megakernel's colour bit for bit."""
+    import torch
+    from pltfalcor_amd.bsdf import default_context
+    from pltfalcor_amd.pltpt import PLTPT
+    from pltfalcor_amd.scene import Scene
+    from test_env_map import _patchy_sky
+    from test_lights import _all_lights
+    ctx = default_context()
+    s = Scene(ctx, seed=41, sphere_count=16, subdivision=3, material_kinds=8)
+    s.set_env_map(_patchy_sky(), rotation=(0.0, 45.0, 0.0), intensity=0.5)
+    s.set_lights(_all_lights())
+    w, h = 1280, 960
+    opts = dict(BASE_OPTS, maxBounces=8, doMNEE=1)
+    ref, _ = _solve_frames(ctx, s, w, h, opts, solve_schedule=PLTPT.SOLVE_MEGAKERNEL)
+    got, st = _solve_frames(ctx, s, w, h, opts, solve_schedule=PLTPT.SOLVE_SPLIT)
+    regions = w * h // 64
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    per = min(64, regions // cus)
+    print(st, "events per block", st["events"] * per / regions)
+    assert per > 1 and st["events"] * per > 4096 * regions and st["walks"] > 0
+    diff = (ref[0] != got[0]).any(axis=2)
+    assert not diff.any(), (int(diff.sum()), np.argwhere(diff)[:5])

@@ -216,3 +216,38 @@ def test_gpu_trace_bit_exact_on_a_deep_tree(gpu):
         ga = t.trace(torch.from_numpy(rr).cuda(), any_hit=True).cpu().numpy()
         assert np.array_equal(ga.astype(np.uint32), O.trace(pos, idx, rr, any_hit=True, brute=True))
     assert (g[0] != 0xFFFFFFFF).mean() > 0.05
+
+
+@pytest.mark.gpu
+def test_gpu_trace_bit_exact_on_a_deep_large_tree(gpu):
+    """The staircase beside 40,000 other triangles: a deep tree above the small-tree rule, so that the loop
+    of larger trees casts closest hits with a deep stack (three entries a level, 32 of them in LDS)."""
+    import torch
+    from pltfalcor_amd.bsdf import Context
+    from pltfalcor_amd.scene import Scene
+    a, base, pos, nrm, idx = _staircase()
+    rng = np.random.default_rng(21)
+    m = 40_000
+    c = rng.uniform(-40, 0, (m, 1, 3))
+    far = (c + rng.uniform(-.5, .5, (m, 3, 3))).astype(np.float32).reshape(-1, 3)
+    idx = np.concatenate([idx, len(pos) + np.arange(3 * m, dtype=np.uint32).reshape(m, 3)])
+    pos = np.concatenate([pos, far])
+    nrm = np.concatenate([nrm, np.tile(np.float32([1, 0, 0]), (3 * m, 1))])
+    t = Scene.from_arrays(Context(0), pos, nrm, idx, np.zeros(len(idx), np.uint32), np.zeros(1, np.uint32), a["materials"],
+                          a["profiles"], base.arrays.camera)
+    info = t.bvh_info()
+    assert info["n_nodes"] >= 4096 and 3 * info["max_depth"] > 32, info
+    n = 8192
+    s = pos[0:900:3, 0]
+    tgt = np.stack([rng.choice(s, n) * rng.uniform(1.0, 1.001, n), rng.uniform(0, 0.2, n) * s[-1], rng.uniform(0, 0.2, n) * s[-1]], 1)
+    o = np.stack([np.full(n, -50.0), tgt[:, 1] * 0.5, tgt[:, 2] * 0.5], 1)
+    o[:n // 2, 1:] = rng.uniform(-40, 0, (n // 2, 2))
+    d = (tgt - o).astype(np.float32)
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    rays = np.ascontiguousarray(np.concatenate([o.T, d.T, np.zeros((1, n)), np.full((1, n), 3.4e38)]), dtype=np.float32)
+    for rr in (rays, random_rays(8192, 12, lo=-40, hi=1e3)):
+        g = t.trace(torch.from_numpy(rr).cuda()).cpu().numpy().view(np.uint32)
+        assert np.array_equal(g, O.trace(pos, idx, rr))
+        assert (g[0] != 0xFFFFFFFF).mean() > 0.05
+        ga = t.trace(torch.from_numpy(rr).cuda(), any_hit=True).cpu().numpy()
+        assert np.array_equal(ga.astype(np.uint32), O.trace(pos, idx, rr, any_hit=True))

@@ -670,7 +670,7 @@ int plt_pass_get_surrogate_stats(plt_pass* pass, uint64_t* rows, uint64_t* exact
  * HWSS components a beam does not carry are not written) to host memory, for analysing which
  * inputs leave the training box; *rows receives the number copied. */
 int plt_pass_copy_surrogate_queries(plt_pass* pass, float* dst, uint64_t max_rows, uint64_t* rows);
-/* The matrix-core GEMM the MLP is built from: C [M x N] (FP32) = A [M x K] * Bt [N x K]^T with
+/* A plain matrix-core GEMM: C [M x N] (FP32) = A [M x K] * Bt [N x K]^T with
  * bf16 row-major operands, K a multiple of 32 (for tests of the kernel). */
 int plt_mlp_gemm_nt(uint32_t M, uint32_t N, uint32_t K, const void* A, const void* Bt, float* C, plt_stream stream);
 

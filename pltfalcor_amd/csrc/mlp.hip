@@ -29,7 +29,8 @@ constexpr int kParams = kHid * kIn + kHid + 2 * (kHid * kHid + kHid) + kOut * kH
 static_assert(kParams == 38032, "parameter count");
 
 // ---------------------------------------------------------------------------------------
-// Plain NT GEMM, C[M x N] = A[M x K] * Bt[N x K]^T (plt_mlp_gemm_nt).
+// Plain NT GEMM, C[M x N] = A[M x K] * Bt[N x K]^T, the entry point plt_mlp_gemm_nt; neither training nor
+// inference uses it.
 // ---------------------------------------------------------------------------------------
 struct GemmArgs {
     const __bf16* A;   // [M x K]
@@ -89,7 +90,7 @@ __global__ void __launch_bounds__(kGemmThreads) gemm_nt_kernel(GemmArgs g) {
 
 int gemm(const GemmArgs& g, hipStream_t st) {
     if (g.M <= 0 || g.N <= 0 || g.K <= 0 || g.K % kKStep)
-        return set_error(PLT_EINVAL, "mlp gemm: shapes must be multiples of 32 (K) and 8 (leading dimensions)");
+        return set_error(PLT_EINVAL, "mlp gemm: shapes must be positive, K a multiple of 32");
     const dim3 grid((g.N + kTile - 1) / kTile, (g.M + kTile - 1) / kTile);
     hipLaunchKernelGGL(gemm_nt_kernel, grid, dim3(kGemmThreads), 0, st, g);
     return check_launch("gemm_nt_kernel");

@@ -105,9 +105,9 @@ __host__ __device__ inline uint32_t path_pixel(uint32_t width, uint32_t height, 
 // Split solve pass. The light-sampling kernel (one 64-lane wave per region of 64 consecutive paths)
 // replays each path's vertices with the path's random stream -- light samples, shadow rays and
 // manifold walks -- and appends one light event per sourced beam that reaches the vertex: NEE,
-// emissive hit or environment miss. The unwind kernel (one wave per region) rebuilds each beam,
-// carries it through the stored vertices to the camera and sums every path's events in the order
-// the megakernel adds them. Events are SoA planes of kEvWords words; a region's events occupy
+// emissive hit or environment miss. The unwind kernels rebuild each beam and carry it through the
+// stored vertices to the camera, and the sum kernel adds every path's events in the order the megakernel
+// adds them. Events are SoA planes of kEvWords words; a region's events occupy
 // [region * 64 * ev_per_path, +64 * ev_per_path) in the order they were appended, which is each
 // path's own vertex order. Walk vertices of manifold NEE events live in a second area, kHitWords
 // planes per vertex, 64 * hits_per_path per region.

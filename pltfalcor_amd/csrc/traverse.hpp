@@ -152,14 +152,16 @@ __device__ __forceinline__ uint32_t box_key(float entry, uint32_t slot) {
 // change the speed: the closest hit is the smallest (t, triangle id) over every triangle tested,
 // and boxes are conservative).
 //
-// A wave issues the instructions of its slowest lanes: 9 to 13 of 64 lanes are active on average in
-// the frame's kernels, which are bound by VALU issue (70-80 % busy). So a trip is kept short and
+// A wave issues the instructions of its slowest lanes: 9 to 14 of 64 lanes are active on average in
+// the frame's kernels, which are bound by VALU issue (70-84 % busy). So a trip is kept short and
 // fits every lane: each lane reads 112 B, the boxes of its node or two triangles of its leaf, with
 // one wait for both kinds (a leaf of four takes two trips, during which the other lanes advance,
 // instead of the wave waiting for its longest leaf), and the hit children are pushed without
 // branches. Against one node or one whole leaf per trip: 1,048,576 incoherent closest-hit rays over
-// 1.31 M triangles 0.413 -> 0.394 ms; per 1080p frame of 5.24 M triangles sample kernel 2.80 -> 2.66,
-// light sampling 2.74 -> 2.63 ms. (The two loads apart, with one triangle per trip: 0.46 ms.)
+// 1.31 M triangles 0.421 -> 0.380 ms; per 1080p frame of 5.24 M triangles sample kernel 2.78 -> 2.63,
+// light sampling 2.72 -> 2.63 ms. (The two loads apart, with one triangle per trip: 0.46 ms.) The ray's
+// constants and the slab test stand in the function itself: taken from RayConst and box_entry, as
+// traverse_quad does, the compiler moved the loads into the branches (0.48 ms).
 template <int kDepth>
 __device__ __forceinline__ Hit traverse_rays(const TraceScene& sc, const Ray& r, int* stack, int stride, bool anyHit) {
     Hit h{kNoHit, 0.f, 0.f, r.tmax};
